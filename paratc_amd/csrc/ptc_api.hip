@@ -311,7 +311,7 @@ int channel_step(ptc_ctx *c, double *mon) {
       PTC_TRY(stencil_prepare(c));  // partials for the x pass's workgroups (already sized under capture)
       const DivSrc dv{ux, uy, uz, 1.0 / c->pmAlpha, c->d_red};
       PTC_TRY(poisson_solve_div(c, dv, hl, true));
-      if (ns == c->iadvance) PTC_TRY(launch_divmax(c, (int)fft2_x_fwd_blocks(c, c->ny)));
+      if (ns == c->iadvance) PTC_TRY(launch_divmax(c, (int)fft_x_fwd_blocks(c, c->ny)));
     } else {
       PTC_TRY(launch_prsrc(c, ux, uy, uz, a1, nullptr, ns == c->iadvance));
       PTC_TRY(poisson_solve(c, a1, hl, true));
@@ -437,8 +437,8 @@ int prepare_step(ptc_ctx *c) {
     PTC_TRY(field(c, f, &d));
   if (c->prm.scalar)
     for (int f : {PTC_F_SCALAR, PTC_F_HISTC, PTC_F_ARRC}) PTC_TRY(field(c, f, &d));
-  PTC_TRY(stencil_prepare(c));
   PTC_TRY(poisson_prepare(c));
+  PTC_TRY(stencil_prepare(c));  // sized by the plan's x pass
   PTC_HIP(hipStreamSynchronize(c->stream));
   return PTC_OK;
 }

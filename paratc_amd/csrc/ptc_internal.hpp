@@ -71,14 +71,17 @@ struct Geo {
 };
 
 // One complex FFT length: radix plan and twiddle table w^m = exp(-2 pi i m / n).
+// Stage s: radix, span (product of the radices before it), the 32-bit
+// reciprocal of the span, and the twiddle step n / (span radix).
+constexpr int kFftMaxStages = 6;
 struct FftLen {
   int n;
   int nstage;
-  int radix[16];
+  int threads;  // threads per line: n / smallest radix
+  int radix[kFftMaxStages], span[kFftMaxStages], step[kFftMaxStages];
+  unsigned magic[kFftMaxStages];
   const double2 *tw;
 };
-
-constexpr int kMaxRadix = 8;
 
 struct PoissonPlan {
   bool ready = false;
@@ -95,9 +98,10 @@ struct PoissonPlan {
   int ztile = 4;      // columns per z-FFT workgroup in use
   int zfast_req = 0;  // column tile of the specialised z kernel (0 = its default)
   bool x_fast = false, z_fast = false;  // compile-time specialised FFT kernels in use
-  int z_threads = 256;
-  int x_lines = 4;    // lines per x-FFT workgroup
+  int x_lines = 4;    // run-time length x pass: lines per workgroup, its threads, LDS padding shift and bytes
   int x_threads = 256;
+  int x_pad = 3;
+  size_t x_lds = 0;
   int tri_chunks = 1; // chunks (waves) per line in the partitioned solver
   int tri_mmax = 16;  // register rows per thread (chunk length)
   int tri_lpb = 64;   // lines per workgroup
@@ -243,8 +247,8 @@ int poisson_build_plan(ptc_ctx *c);
 int poisson_free_plan(ptc_ctx *c);
 // ghosts: also fill dst's Neumann ghost rows j = 0, ny+1 (SetBC_and_UpdateHalo_pr)
 int poisson_solve(ptc_ctx *c, const double *src, double *dst, bool ghosts = false);
-// clcPrSrc + clcPPE with the source formed in the x pass (FP64 plans with the
-// specialised x kernel and no slabs: poisson_div_fusable)
+// clcPrSrc + clcPPE with the source formed in the x pass (FP64 plans without
+// slabs: poisson_div_fusable)
 bool poisson_div_fusable(ptc_ctx *c);
 int poisson_solve_div(ptc_ctx *c, const DivSrc &div, double *dst, bool ghosts);
 int poisson_prepare(ptc_ctx *c);
@@ -287,6 +291,10 @@ int poisson_stage_times(ptc_ctx *c, float *ms5, int *nsolves);
 int launch_fft_x_fwd(ptc_ctx *c, const double *src, void *spec, bool f64 = false);
 int launch_fft_x_inv(ptc_ctx *c, const void *spec, double *dst, double scale, bool acc, bool ghost);
 int launch_fft_z(ptc_ctx *c, void *spec, bool inverse, bool f64 = false);
+// the x forward pass with the Poisson source formed from the velocities (FP64 spectra)
+int launch_fft_x_fwd_div(ptc_ctx *c, const DivSrc &div, void *spec);
+// workgroups of one x forward launch over nj planes with the plan in use
+long long fft_x_fwd_blocks(const ptc_ctx *c, int nj);
 int fft_make_len(int n, FftLen *L);
 bool fft2_has_x(int h);
 bool fft2_has_z(int nz, int req, int *tile);

@@ -28,7 +28,8 @@
 
 namespace ptc {
 
-bool fft_config_ok(const FftLen &L, int ncol, int nthr);
+bool fft_x_shape(const FftLen &L, size_t lds_cap, int *lines, int *threads, int *pad, size_t *lds);
+int fft_z_tile(const FftLen &L, size_t lds_cap, int most);
 int tri_plan(int ny, size_t lds_limit, bool poisson, int mm_req, int lpb_req, int *P_out, int *mm_out, int *lpb_out);
 int tri_plan_lds(int ny, size_t lds_limit, int ll, int mm_req, int *P_out, int *mm_out);
 int tri_plan_cplx(int ny, size_t lds_limit, int cl, int mm_req, int *P_out, int *mm_out);
@@ -85,15 +86,9 @@ int poisson_build_plan(ptc_ctx *c) {
   // specialised kernels for the production lengths unless a tile is forced
   P.x_fast = P.ztile_req == 0 && fft2_has_x(P.h);
   if (!P.x_fast) {
-    // generic x pass: lines per workgroup so that a tile holds ~2048 complex values
-    P.x_lines = std::max(1, 2048 / P.h);
-    while (P.x_lines > 1 && sizeof(double2) * (size_t)P.h * P.x_lines > lds_cap) P.x_lines /= 2;
-    PTC_CHECK(sizeof(double2) * (size_t)P.h * P.x_lines <= lds_cap, PTC_E_UNSUPPORTED,
-              "nx too large for the LDS x-FFT");
-    P.x_threads = 0;
-    for (int t : {256, 512, 1024})
-      if (fft_config_ok(P.fx, P.x_lines, t)) { P.x_threads = t; break; }
-    PTC_CHECK(P.x_threads > 0, PTC_E_UNSUPPORTED, "no x-FFT launch shape fits");
+    PTC_CHECK(sizeof(double2) * (size_t)P.h <= lds_cap, PTC_E_UNSUPPORTED, "nx too large for the LDS x-FFT");
+    PTC_CHECK(fft_x_shape(P.fx, lds_cap, &P.x_lines, &P.x_threads, &P.x_pad, &P.x_lds), PTC_E_UNSUPPORTED,
+              "no x-FFT launch shape fits");
   }
 
   int zt = 0;
@@ -101,16 +96,12 @@ int poisson_build_plan(ptc_ctx *c) {
   if (P.z_fast) {
     P.ztile = zt;
   } else {
-    // generic z pass: widest column tile (<= 16, divides pitch) that fits LDS
-    int T = P.ztile_req > 0 ? P.ztile_req : 16;
-    while (T > 1 && (sizeof(double2) * (size_t)c->nz * T > lds_cap || (size_t)T * c->nz > 4096)) T /= 2;
+    // run-time length z pass: widest column tile (<= 16, divides pitch) that fits
+    const int T = fft_z_tile(P.fz, lds_cap, P.ztile_req > 0 ? P.ztile_req : 16);
     PTC_CHECK(P.pitch % T == 0, PTC_E_ARG, "z tile must divide the spectral pitch");
     PTC_CHECK(sizeof(double2) * (size_t)c->nz * T <= lds_cap, PTC_E_UNSUPPORTED, "nz too large for the LDS z-FFT");
+    PTC_CHECK(P.fz.threads * T <= 1024, PTC_E_UNSUPPORTED, "no z-FFT launch shape fits");
     P.ztile = T;
-    P.z_threads = 0;
-    for (int t : {256, 512, 1024})
-      if (fft_config_ok(P.fz, T, t)) { P.z_threads = t; break; }
-    PTC_CHECK(P.z_threads > 0, PTC_E_UNSUPPORTED, "no z-FFT launch shape fits");
   }
 
   // x/z passes over slabs of y planes (specialised kernels only): the z pass
@@ -228,7 +219,7 @@ static int solve_sequence(ptc_ctx *c, const double *src, double *dst, bool acc, 
   PoissonPlan &P = c->pp;
   if (ev) PTC_HIP(hipEventRecord(ev[0], c->stream));
   if (div) {
-    PTC_TRY(fft2_x_fwd(c, nullptr, P.d_spec, 0, c->ny, false, div));
+    PTC_TRY(launch_fft_x_fwd_div(c, *div, P.d_spec));
     if (ev) PTC_HIP(hipEventRecord(ev[1], c->stream));
     PTC_TRY(launch_fft_z(c, P.d_spec, false));
   } else if (res && P.slab == 0) {
@@ -311,14 +302,15 @@ int poisson_solve(ptc_ctx *c, const double *src, double *dst, bool ghosts) {
 bool poisson_div_fusable(ptc_ctx *c) {
   if (poisson_build_plan(c) != PTC_OK) return false;
   const PoissonPlan &P = c->pp;
-  return P.x_fast && P.slab == 0 && P.prec == PTC_PREC_FP64;
+  // (a run-time length plan with a radix above 10 has no registers left for it)
+  return P.slab == 0 && P.prec == PTC_PREC_FP64 && (P.x_fast || P.fx.radix[0] <= 10);
 }
 
 int poisson_solve_div(ptc_ctx *c, const DivSrc &div, double *dst, bool ghosts) {
   PTC_TRY(poisson_build_plan(c));
   PoissonPlan &P = c->pp;
-  PTC_CHECK(P.x_fast && P.slab == 0 && P.prec == PTC_PREC_FP64, PTC_E_STATE,
-            "the divergence-forming solve needs an FP64 plan with the specialised x pass and no slabs");
+  PTC_CHECK(poisson_div_fusable(c), PTC_E_STATE,
+            "the divergence-forming solve needs an FP64 plan without slabs whose x pass can form it");
   PTC_TRY(ensure_thomas_scratch(c));
   hipEvent_t *ev = nullptr;
   if (P.profile) {

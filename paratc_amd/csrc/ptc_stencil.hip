@@ -1121,7 +1121,7 @@ int flow_fold(ptc_ctx *c, bool first, FlowFold *ff) {
 // reduction partials of the RHS and PrSrc kernels, allocated ahead of a
 // captured step
 int stencil_prepare(ptc_ctx *c) {
-  const int nx = (int)fft2_x_fwd_blocks(c, c->ny);
+  const int nx = (int)fft_x_fwd_blocks(c, c->ny);
   return ensure_red(c, std::max({pt_nblocks(c), rhs_nblocks(c), nx}));
 }
 
