@@ -259,6 +259,20 @@ static int step_cn_jobs(ptc_ctx *c, CnJobs *cn) {
   return PTC_OK;
 }
 
+// The monitors after a step into mon[0..4], one pass and one wait; cfl: also
+// 0.5 times the CFL maximum launched before the step into mon[5]
+static int step_monitors(ptc_ctx *c, const double *ux, const double *uy, const double *uz, bool cfl, double *mon) {
+  Monitors mo{};
+  PTC_TRY(launch_monitors(c, kMonDiv | kMonVmax, ux, uy, uz));
+  PTC_TRY(read_monitors(c, kMonDiv | kMonVmax | (cfl ? kMonCfl : 0), &mo));
+  mon[0] = mo.div_prsrc;
+  c->divmax_prsrc = mo.div_prsrc;
+  mon[1] = mo.div;
+  for (int q = 0; q < 3; ++q) mon[2 + q] = mo.v[q];
+  if (cfl) mon[5] = 0.5 * mo.cfl;
+  return PTC_OK;
+}
+
 int channel_step(ptc_ctx *c, double *mon) {
   double *ux, *uy, *uz, *p, *hx, *hy, *hz, *a1, *a2, *hl, *uym, *duym;
   double *sc = nullptr, *hc = nullptr, *ac = nullptr;
@@ -280,14 +294,17 @@ int channel_step(ptc_ctx *c, double *mon) {
     PTC_TRY(field(c, PTC_F_HISTC, &hc));
     PTC_TRY(field(c, PTC_F_ARRC, &ac));
   }
-  // CalcMaxCFL and dt (:93-100)
-  double cflmp = 0.0, dt = c->prm.dtmax;
-  if (c->prm.icfl == 1 || mon) {
-    double uddxmax = 0.0;
-    PTC_TRY(launch_monitor(c, 0, ux, uy, uz, nullptr, &uddxmax));
-    uddxmax *= 0.5;
-    cflmp = uddxmax * c->dt;
-    if (c->prm.icfl == 1) dt = std::min(c->prm.cflc / uddxmax, c->prm.dtmax);
+  // CalcMaxCFL and dt (:93-100): only an adaptive dt needs the value before
+  // the step, else it is read with the other monitors after it
+  const double dt_old = c->dt;
+  double dt = c->prm.dtmax, uddxmax = 0.0;
+  Monitors mo{};
+  const bool adaptive = c->prm.icfl == 1;
+  if (adaptive || mon) PTC_TRY(launch_monitors(c, kMonCfl, ux, uy, uz));
+  if (adaptive) {
+    PTC_TRY(read_monitors(c, kMonCfl, &mo));
+    uddxmax = 0.5 * mo.cfl;
+    dt = std::min(c->prm.cflc / uddxmax, c->prm.dtmax);
   }
   // constant flow rate: the Crank-Nicolson launch sums the RHS kernel's
   // flow-rate partials itself (no k_flowrate launch, no PrGradAver zeroing)
@@ -321,13 +338,9 @@ int channel_step(ptc_ctx *c, double *mon) {
     PTC_TRY(launch_vel_p_update_bc(c, hl, ux, uy, uz, p, uym));
   }
   if (mon) {
-    PTC_TRY(get_device_scalar(c, S_DIVMAX, &mon[0]));
-    c->divmax_prsrc = mon[0];
-    PTC_TRY(launch_monitor(c, 1, ux, uy, uz, nullptr, &mon[1]));
-    PTC_TRY(launch_monitor(c, 2, ux, uy, uz, nullptr, &mon[2]));
-    PTC_TRY(launch_monitor(c, 3, ux, uy, uz, nullptr, &mon[3]));
-    PTC_TRY(launch_monitor(c, 4, ux, uy, uz, nullptr, &mon[4]));
-    mon[5] = cflmp;
+    PTC_TRY(step_monitors(c, ux, uy, uz, !adaptive, mon));
+    if (adaptive) mon[5] = uddxmax * dt_old;
+    else mon[5] *= dt_old;
     mon[6] = dt;
   }
   return PTC_OK;
@@ -404,27 +417,18 @@ static int graph_step(ptc_ctx *c, double *mon) {
     PTC_TRY(capture_step(c, &c->step_graph, &c->step_exec));
     c->step_gen = c->buf_gen;
   }
-  double cflmp = 0.0;
   double *ux, *uy, *uz;
   PTC_TRY(field(c, PTC_F_UX, &ux));
   PTC_TRY(field(c, PTC_F_UY, &uy));
   PTC_TRY(field(c, PTC_F_UZ, &uz));
-  if (mon) {
-    double uddxmax = 0.0;
-    PTC_TRY(launch_monitor(c, 0, ux, uy, uz, nullptr, &uddxmax));
-    cflmp = 0.5 * uddxmax * c->dt;
-  }
+  const double dt_old = c->dt;
+  if (mon) PTC_TRY(launch_monitors(c, kMonCfl, ux, uy, uz));
   PTC_HIP(hipGraphLaunch(c->step_exec, c->stream));
   c->dt = c->prm.dtmax;
   c->simtime += c->prm.dtmax;  // the RK3 alphas sum to one
   if (mon) {
-    PTC_TRY(get_device_scalar(c, S_DIVMAX, &mon[0]));
-    c->divmax_prsrc = mon[0];
-    PTC_TRY(launch_monitor(c, 1, ux, uy, uz, nullptr, &mon[1]));
-    PTC_TRY(launch_monitor(c, 2, ux, uy, uz, nullptr, &mon[2]));
-    PTC_TRY(launch_monitor(c, 3, ux, uy, uz, nullptr, &mon[3]));
-    PTC_TRY(launch_monitor(c, 4, ux, uy, uz, nullptr, &mon[4]));
-    mon[5] = cflmp;
+    PTC_TRY(step_monitors(c, ux, uy, uz, true, mon));
+    mon[5] *= dt_old;
     mon[6] = c->prm.dtmax;
   }
   return PTC_OK;
@@ -881,8 +885,10 @@ int ptc_calc_max_cfl(ptc_ctx *ctx, int ux, int uy, int uz, double *out) {
   PTC_CHECK(out, PTC_E_ARG, "null output");
   double *u, *v, *w;
   PTC_TRY(three(ctx, ux, uy, uz, &u, &v, &w));
-  PTC_TRY(launch_monitor(ctx, 0, u, v, w, nullptr, out));
-  *out *= 0.5;
+  Monitors mo{};
+  PTC_TRY(launch_monitors(ctx, kMonCfl, u, v, w));
+  PTC_TRY(read_monitors(ctx, kMonCfl, &mo));
+  *out = 0.5 * mo.cfl;
   return PTC_OK;
 }
 
@@ -891,7 +897,11 @@ int ptc_check_divergence(ptc_ctx *ctx, int ux, int uy, int uz, double *out) {
   PTC_CHECK(out, PTC_E_ARG, "null output");
   double *u, *v, *w;
   PTC_TRY(three(ctx, ux, uy, uz, &u, &v, &w));
-  return launch_monitor(ctx, 1, u, v, w, nullptr, out);
+  Monitors mo{};
+  PTC_TRY(launch_monitors(ctx, kMonDiv, u, v, w));
+  PTC_TRY(read_monitors(ctx, kMonDiv, &mo));
+  *out = mo.div;
+  return PTC_OK;
 }
 
 int ptc_calc_vmax(ptc_ctx *ctx, int ux, int uy, int uz, double *v3) {
@@ -899,7 +909,10 @@ int ptc_calc_vmax(ptc_ctx *ctx, int ux, int uy, int uz, double *v3) {
   PTC_CHECK(v3, PTC_E_ARG, "null output");
   double *u, *v, *w;
   PTC_TRY(three(ctx, ux, uy, uz, &u, &v, &w));
-  for (int q = 0; q < 3; ++q) PTC_TRY(launch_monitor(ctx, 2 + q, u, v, w, nullptr, &v3[q]));
+  Monitors mo{};
+  PTC_TRY(launch_monitors(ctx, kMonVmax, u, v, w));
+  PTC_TRY(read_monitors(ctx, kMonVmax, &mo));
+  for (int q = 0; q < 3; ++q) v3[q] = mo.v[q];
   return PTC_OK;
 }
 
@@ -908,7 +921,7 @@ int ptc_calc_ux_aver(ptc_ctx *ctx, int ux, double *mean) {
   PTC_CHECK(mean, PTC_E_ARG, "null output");
   double *u;
   PTC_TRY(field(ctx, ux, &u));
-  PTC_TRY(launch_monitor(ctx, 5, u, u, u, nullptr, mean));
+  PTC_TRY(launch_monitor_sum(ctx, 0, u, nullptr, mean));
   *mean = *mean / (double)(ctx->nx * ctx->nz) / ctx->yly;
   return PTC_OK;
 }
@@ -920,7 +933,7 @@ int ptc_clc_mean_value(ptc_ctx *ctx, int ux, int scalar, double *res3) {
   PTC_TRY(field(ctx, ux, &u));
   PTC_TRY(field(ctx, scalar, &s));
   for (int q = 0; q < 3; ++q) {
-    PTC_TRY(launch_monitor(ctx, 6 + q, u, u, u, s, &res3[q]));
+    PTC_TRY(launch_monitor_sum(ctx, 1 + q, u, s, &res3[q]));
     res3[q] = res3[q] / (double)(ctx->nx * ctx->nz) / ctx->yly;
   }
   return PTC_OK;

@@ -163,6 +163,7 @@ struct ptc_ctx {
   double *d_red = nullptr;     // reduction partials
   int red_cap = 0;
   double *d_scal = nullptr;    // device scalars
+  double *d_mon = nullptr;     // partial maxima of the monitors
   double *d_cnfac = nullptr;   // Crank-Nicolson factor tables (kCnMaxJobs + kCnStepTables) x kCnFacStride
   // beta each step table (substep ns, kind) holds, NaN when none; the tables
   // also depend on the chunk plan (cn_tab_mm, cn_tab_p) and the metrics
@@ -414,8 +415,16 @@ int launch_bc_scalar(ptc_ctx *c, double *s);
 int launch_visu(ptc_ctx *c, int which, const double *ux, const double *uy, const double *uz, const double *p,
                 const double *sc, int iskip, int jskip, int kskip, int real_bytes, void *dev_out);
 int launch_uy_ym(ptc_ctx *c, double *uy_ym, double *duy_ym);
-int launch_monitor(ptc_ctx *c, int which, const double *ux, const double *uy, const double *uz,
-                   const double *s, double *out);
+// The monitors of a step: launch_monitors enqueues one pass over the velocities
+// for a set of maxima, read_monitors waits and returns them (h_pinned + kPinMonitors).
+constexpr int kMonCfl = 1, kMonDiv = 2, kMonVmax = 4;
+constexpr int kPinMonitors = 16;
+struct Monitors {
+  double cfl, div, v[3], div_prsrc;
+};
+int launch_monitors(ptc_ctx *c, int what, const double *ux, const double *uy, const double *uz);
+int read_monitors(ptc_ctx *c, int what, Monitors *out);
+int launch_monitor_sum(ptc_ctx *c, int which, const double *ux, const double *s, double *out);
 int reduce_sum_s3(ptc_ctx *c, int nparts, double *host_out);
 
 // The partial results of a launch reduced by one workgroup of

@@ -892,46 +892,126 @@ int launch_visu(ptc_ctx *c, int which, const double *ux, const double *uy, const
 }
 
 // ---- monitors (m_Tools) -------------------------------------------------------
-// which: 0 CFL max (:24-49), 1 divergence max (:54-81), 2..4 |ux|,|uy|,|uz| max (:86-110),
-//        5 sum ux*dyp (:256-275), 6..8 sums dyp*(ux, c, c^2) (:281-301)
-__global__ void __launch_bounds__(256) k_monitor(Geo g, int which, const double *__restrict__ ux,
-                                                const double *__restrict__ uy, const double *__restrict__ uz,
-                                                const double *__restrict__ sc, double *__restrict__ part) {
+// The maxima of a step: CFL sum (:24-49), |divergence| (:54-81) and |ux|, |uy|,
+// |uz| (:86-110), as many of them as the instantiation asks for in one pass over
+// the velocities.  Bound by memory: 24 B per point however many are formed (one
+// pass each took 6 x 357 us a step at 1536x192x256).  As k_vel_p_update, a 64 x 4
+// tile marches k over a chunk of planes with uz's window in registers and the
+// next plane's loads issued before the current plane is formed.  Lanes past nx
+// and rows past ny repeat the last point, which changes no maximum.  Workgroup
+// maxima of quantity q (0 CFL, 1 divergence, 2..4 velocities) go to
+// part[q nb + workgroup].
+constexpr int kMonitors = 5;
+
+template <bool CFL, bool DIV, bool VMAX>
+__global__ void __launch_bounds__(256) k_monitors(Geo g, const double *__restrict__ ux, const double *__restrict__ uy,
+                                                 const double *__restrict__ uz, int kc, int run,
+                                                 double *__restrict__ part) {
+  __shared__ double sh[4][kMonitors];
+  const int nwg = (int)(gridDim.x * gridDim.y * gridDim.z);
+  const int wt = xcd_run((int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)), nwg, run);
+  const int by = wt % (int)gridDim.y, bx = (wt / (int)gridDim.y) % (int)gridDim.x,
+            bz = wt / (int)(gridDim.x * gridDim.y);
+  const int nx = g.nx, nz = g.nz;
+  const int i = min(bx * 64 + (int)threadIdx.x, nx - 1), j = min(by * 4 + (int)threadIdx.y + 1, g.ny);
+  const int k0 = bz * kc, k1 = min(k0 + kc, nz);
+  const int im1 = wrapi(i - 1, nx), ip1 = wrapi(i + 1, nx), ip2 = wrapi(i + 2, nx);
+  const long long rj = (long long)nx * j;
+  const double rdyp = g.met[M_RDYP * g.nyh + j];
+  struct Plane {
+    double xm, x, xp, xpp, y, yp;
+  };
+  auto load = [&](int k) {
+    const long long o = rj + (long long)k * g.plane;
+    Plane q{};
+    q.x = ux[o + i];
+    q.y = uy[o + i];
+    if (CFL || DIV) {
+      q.xp = ux[o + ip1];
+      q.yp = uy[o + nx + i];
+    }
+    if (DIV) {
+      q.xm = ux[o + im1];
+      q.xpp = ux[o + ip2];
+    }
+    return q;
+  };
+  auto wz = [&](int kk) { return uz[i + rj + (long long)wrapi(kk, nz) * g.plane]; };
+  double w0 = DIV ? wz(k0 - 1) : 0.0, w1 = wz(k0), w2 = wz(k0 + 1);
+  double m[kMonitors] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  Plane cur = load(k0);
+  for (int k = k0; k < k1; ++k) {
+    const Plane nxt = load(k + 1 < k1 ? k + 1 : k);
+    const double w3 = wz(k + 2);
+    if (CFL)
+      m[0] = fmax(m[0], fabs(cur.x + cur.xp) * g.rdx + fabs(cur.y + cur.yp) * rdyp + fabs(w1 + w2) * g.rdz);
+    if (DIV) {
+      const double dudx = g.dxc1 * cur.xm + g.dxc2 * cur.x + g.dxc3 * cur.xp + g.dxc4 * cur.xpp;
+      const double dvdy = (cur.yp - cur.y) * rdyp;
+      const double dwdz = g.dzc1 * w0 + g.dzc2 * w1 + g.dzc3 * w2 + g.dzc4 * w3;
+      m[1] = fmax(m[1], fabs(dudx + dvdy + dwdz));
+    }
+    if (VMAX) {
+      m[2] = fmax(m[2], fabs(cur.x));
+      m[3] = fmax(m[3], fabs(cur.y));
+      m[4] = fmax(m[4], fabs(w1));
+    }
+    cur = nxt;
+    w0 = w1;
+    w1 = w2;
+    w2 = w3;
+  }
+  constexpr int q0 = CFL ? 0 : (DIV ? 1 : 2), q1 = VMAX ? 5 : (DIV ? 2 : 1);
+#pragma unroll
+  for (int q = q0; q < q1; ++q) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m[q] = fmax(m[q], __shfl_xor(m[q], off));
+    if (threadIdx.x == 0) sh[threadIdx.y][q] = m[q];
+  }
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (threadIdx.y == 0 && t >= q0 && t < q1)
+    part[(long long)t * nwg + wt] = fmax(fmax(sh[0][t], sh[1][t]), fmax(sh[2][t], sh[3][t]));
+}
+
+// The maxima of quantities q0 .. q0 + gridDim.x - 2 over their nb partials, and
+// (last workgroup) the divergence maximum of clcPrSrc, straight into host memory
+// the device can write: the caller waits once and reads them all.
+__global__ void __launch_bounds__(kReduceThreads) k_final_monitors(const double *__restrict__ part, int nb, int q0,
+                                                                  const double *__restrict__ scal,
+                                                                  double *__restrict__ host) {
+  if (blockIdx.x + 1 == gridDim.x) {
+    if (threadIdx.x == 0) host[kMonitors] = scal[S_DIVMAX];
+    return;
+  }
+  const int q = q0 + (int)blockIdx.x;
+  const double t = reduce_partials<true>(part + (long long)q * nb, nb);
+  if (threadIdx.x == 0) host[q] = t;
+}
+
+// which: 0 sum ux*dyp (:256-275), 1..3 sums dyp*(ux, c, c^2) (:281-301)
+__global__ void __launch_bounds__(256) k_monitor_sum(Geo g, int which, const double *__restrict__ ux,
+                                                    const double *__restrict__ sc, double *__restrict__ part) {
   __shared__ double sh[256];
   const int i = blockIdx.x * 64 + threadIdx.x;
   const int j = blockIdx.y * 4 + threadIdx.y + 1;
   const int k = blockIdx.z;
   double v = 0.0;
   if (i < g.nx && j <= g.ny) {
-    const Ngh N(g, i, k);
-    const int W = g.nyh;
+    const long long o = i + (long long)g.nx * j + g.plane * k;
+    const double dyp = g.met[M_DYP * g.nyh + j];
     switch (which) {
       case 0:
-        v = fabs(N(ux, 0, j, 0) + N(ux, 1, j, 0)) * g.rdx + fabs(N(uy, 0, j, 0) + N(uy, 0, j + 1, 0)) * g.met[M_RDYP * W + j] +
-            fabs(N(uz, 0, j, 0) + N(uz, 0, j, 1)) * g.rdz;
-        break;
-      case 1: {
-        const double dudx = g.dxc1 * N(ux, -1, j, 0) + g.dxc2 * N(ux, 0, j, 0) + g.dxc3 * N(ux, 1, j, 0) +
-                            g.dxc4 * N(ux, 2, j, 0);
-        const double dvdy = (N(uy, 0, j + 1, 0) - N(uy, 0, j, 0)) * g.met[M_RDYP * W + j];
-        const double dwdz = g.dzc1 * N(uz, 0, j, -1) + g.dzc2 * N(uz, 0, j, 0) + g.dzc3 * N(uz, 0, j, 1) +
-                            g.dzc4 * N(uz, 0, j, 2);
-        v = fabs(dudx + dvdy + dwdz);
-      } break;
-      case 2: v = fabs(N(ux, 0, j, 0)); break;
-      case 3: v = fabs(N(uy, 0, j, 0)); break;
-      case 4: v = fabs(N(uz, 0, j, 0)); break;
-      case 5:
-      case 6: v = N(ux, 0, j, 0) * g.met[M_DYP * W + j]; break;
-      case 7: v = g.met[M_DYP * W + j] * N(sc, 0, j, 0); break;
-      case 8: {
-        const double s = N(sc, 0, j, 0);
-        v = g.met[M_DYP * W + j] * s * s;
+      case 1: v = ux[o] * dyp; break;
+      case 2: v = dyp * sc[o]; break;
+      case 3: {
+        const double s = sc[o];
+        v = dyp * s * s;
       } break;
       default: break;
     }
   }
-  const double t = (which <= 4) ? block_max(v, sh) : block_sum(v, sh);
+  const double t = block_sum(v, sh);
   if (threadIdx.x == 0 && threadIdx.y == 0) part[blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)] = t;
 }
 
@@ -1298,17 +1378,54 @@ int launch_uy_ym(ptc_ctx *c, double *uy_ym, double *duy_ym) {
   return launch_bc(c, b, nullptr, nullptr, nullptr, uy_ym, duy_ym);
 }
 
-// result to host (synchronises)
-int launch_monitor(ptc_ctx *c, int which, const double *ux, const double *uy, const double *uz, const double *s,
-                   double *out) {
+// Enqueue the pass over the velocities that forms the asked maxima (kMon...);
+// read_monitors later brings them to the host.  The partials have their own
+// buffer, so a step may run in between.
+int launch_monitors(ptc_ctx *c, int what, const double *ux, const double *uy, const double *uz) {
+  int kc = 0;
+  const dim3 grid = vel_grid(c, &kc);
+  const int nb = (int)(grid.x * grid.y * grid.z);
+  if (!c->d_mon) PTC_HIP(hipMalloc(&c->d_mon, sizeof(double) * (size_t)nb * kMonitors));
+#define PTC_MON(C, D, V)                                                                                      \
+  hipLaunchKernelGGL((k_monitors<C, D, V>), grid, dim3(64, 4), 0, c->stream, c->geo, ux, uy, uz, kc, kVelXcdRun, \
+                     c->d_mon)
+  if (what == kMonCfl) PTC_MON(true, false, false);
+  else if (what == kMonDiv) PTC_MON(false, true, false);
+  else if (what == kMonVmax) PTC_MON(false, false, true);
+  else if (what == (kMonDiv | kMonVmax)) PTC_MON(false, true, true);
+  else PTC_CHECK(false, PTC_E_ARG, "unknown monitor set");
+#undef PTC_MON
+  PTC_HIP(hipGetLastError());
+  return PTC_OK;
+}
+
+// The maxima of `what` (any of the kMon... sets launched since the last read)
+// and clcPrSrc's divergence maximum on the host (synchronises)
+int read_monitors(ptc_ctx *c, int what, Monitors *out) {
+  int kc = 0;
+  const dim3 grid = vel_grid(c, &kc);
+  const int nb = (int)(grid.x * grid.y * grid.z);
+  const int q0 = what & kMonCfl ? 0 : (what & kMonDiv ? 1 : 2);
+  const int q1 = what & kMonVmax ? 5 : (what & kMonDiv ? 2 : 1);
+  double *h = c->h_pinned + kPinMonitors;
+  hipLaunchKernelGGL(k_final_monitors, dim3((unsigned)(q1 - q0 + 1)), dim3(kReduceThreads), 0, c->stream, c->d_mon, nb,
+                     q0, c->d_scal, h);
+  PTC_HIP(hipGetLastError());
+  PTC_HIP(hipStreamSynchronize(c->stream));
+  out->cfl = h[0];
+  out->div = h[1];
+  for (int q = 0; q < 3; ++q) out->v[q] = h[2 + q];
+  out->div_prsrc = h[kMonitors];
+  return PTC_OK;
+}
+
+// a sum to the host (synchronises); which: as k_monitor_sum
+int launch_monitor_sum(ptc_ctx *c, int which, const double *ux, const double *s, double *out) {
   const int nb = pt_nblocks(c);
   PTC_TRY(ensure_red(c, nb));
-  hipLaunchKernelGGL(k_monitor, pt_grid(c), dim3(64, 4), 0, c->stream, c->geo, which, ux, uy, uz, s, c->d_red);
+  hipLaunchKernelGGL(k_monitor_sum, pt_grid(c), dim3(64, 4), 0, c->stream, c->geo, which, ux, s, c->d_red);
   PTC_HIP(hipGetLastError());
-  if (which <= 4)
-    hipLaunchKernelGGL(k_final_max, dim3(1), dim3(kReduceThreads), 0, c->stream, c->d_red, nb, c->d_scal + S_MON0);
-  else
-    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kReduceThreads), 0, c->stream, c->d_red, nb, c->d_scal + S_MON0);
+  hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kReduceThreads), 0, c->stream, c->d_red, nb, c->d_scal + S_MON0);
   PTC_HIP(hipGetLastError());
   PTC_HIP(hipMemcpyAsync(c->h_pinned, c->d_scal + S_MON0, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   PTC_HIP(hipStreamSynchronize(c->stream));
