@@ -1452,80 +1452,200 @@ int get_device_scalar(ptc_ctx *c, int slot, double *out) {
 namespace ptc {
 
 // ---- clcStat (src/m_FlowCase.f90:283-413) ----------------------------------
-// Block (chunk, j): plane j = 1..ny+1, planes k in [chunk*kc, chunk*kc + kc).
-// Each thread sums the reference's SumVec terms over its points; the block
-// reduces them in a fixed order into part[(j-1)][chunk][q].  Plane ny+1 has
-// only the wall terms 27, 33 and 35 (1-based) of the reference.
+// Sums NS values over a wavefront: each of six exchanges sends half of the values
+// a lane still holds to the lane that keeps them, so NS values cost about NS
+// exchanges instead of 6 NS.  On return lane l holds the sum of value *idx in
+// v[0] (*idx = -1: none).  Fixed order.
+template <int NS, int N, int MASK>
+__device__ __forceinline__ void wave_sums_step(double (&v)[NS], int lane, int &base, int &count) {
+  constexpr int H = (N + 1) / 2;
+  const bool up = lane & MASK;
+#pragma unroll
+  for (int q = 0; q < H; ++q) {
+    const double hi = q + H < N ? v[q + H] : 0.0;
+    const double send = up ? v[q] : hi, keep = up ? hi : v[q];
+    v[q] = keep + __shfl_xor(send, MASK);
+  }
+  base += up ? H : 0;
+  count = up ? count - H : min(count, H);
+  if constexpr (MASK > 1) wave_sums_step<NS, H, MASK / 2>(v, lane, base, count);
+}
+template <int NS>
+__device__ __forceinline__ void wave_sums(double (&v)[NS], int lane, int *idx) {
+  static_assert(NS <= 64, "one value per lane at the end");
+  int base = 0, count = NS;
+  wave_sums_step<NS, NS, 32>(v, lane, base, count);
+  *idx = count > 0 ? base : -1;
+}
+
+// The reference's SumVec terms of rows j = 1..ny, marching z as k_rhs_rows does: a
+// workgroup owns rows of x (one thread per column; rows longer than 256 points go
+// in segments of 252 with two wrapped halo columns on either side) and marches
+// k over a chunk of planes.  ux at rows j and j-1, uy and uz at row j sit in
+// register windows k-2..k+2, the other values of a plane are loaded one plane
+// ahead, and the x neighbours (the z difference of uy that dvdzC interpolates
+// included) go through LDS rows, double-buffered so that a plane takes one
+// barrier.  Twelve loads per point instead of about ninety: bound by the loads'
+// latency at the two wavefronts per SIMD that the 40 running sums leave
+// (256x128x192 with a scalar: 563 us a sample before, about 115 now).  part[(j-1) nparts + part][NS]
+// with part = segment * nch + chunk.  The last row group of the grid is the top
+// wall face j = ny+1, which has only the terms 27, 33 and 35 (1-based).
+enum { T_U = 0, T_V, T_VP, T_W, T_P, T_PM, T_C4, T_NROWS };
+
 template <bool SC>
-__global__ void __launch_bounds__(256) k_stat_partial(Geo g, double ucrf, const double *__restrict__ ux,
-                                                      const double *__restrict__ uy, const double *__restrict__ uz,
-                                                      const double *__restrict__ pr, const double *__restrict__ sc,
-                                                      int kc, double *__restrict__ part) {
+__global__ void __launch_bounds__(256, 2) k_stat_rows(Geo g, double ucrf, const double *__restrict__ ux,
+                                                   const double *__restrict__ uy, const double *__restrict__ uz,
+                                                   const double *__restrict__ pr, const double *__restrict__ sc,
+                                                   int kc, int nch, int seg, int lw, int grp,
+                                                   double *__restrict__ part) {
   constexpr int NS = SC ? 40 : 35;
-  __shared__ double sh[256];
-  const int j = blockIdx.y + 1, ny = g.ny;
-  const int k0 = blockIdx.x * kc, k1 = min(k0 + kc, g.nz);
+  extern __shared__ double xr[];
+  __shared__ double wsum[4][NS];
+  const int nx = g.nx, nz = g.nz, ny = g.ny, nyh = g.nyh;
+  const int nyb = (int)gridDim.y, nparts = (int)gridDim.x;
+  const int wt = xcd_run((int)(blockIdx.x + gridDim.x * blockIdx.y), nparts * nyb, grp);
+  const int by = wt % nyb, pt = wt / nyb, bx = pt / nch, ch = pt % nch;  // row groups fastest
+  const int k0 = ch * kc, k1 = min(k0 + kc, nz);
+  const int i = threadIdx.x, nr = (int)blockDim.y, r = (int)threadIdx.y;
+  int gcol = seg ? bx * seg - 2 + i : i;
+  gcol = gcol < 0 ? gcol + nx : (gcol >= nx ? gcol - nx : gcol);
+  const bool own = seg ? (i >= 2 && i < 2 + seg && bx * seg + i - 2 < nx) : i < nx;
+  const bool in = seg ? true : i < nx;
+  const int ic = seg ? min(gcol, nx - 1) : (in ? i : 0);
   const double *met = g.met;
-  const int nyh = g.nyh;
-  const double IY1 = met[M_YINT * nyh + j], IY2 = 1.0 - IY1;
-  const double cac = met[M_RDYC * nyh + j];
   const double I1 = g.ic1, I2 = g.ic2, I3 = g.ic3, I4 = g.ic4;
   const double rdxt = g.rdx / 12.0, rdzt = g.rdz / 12.0;
   double sv[NS];
 #pragma unroll
   for (int q = 0; q < NS; ++q) sv[q] = 0.0;
-  if (j <= ny) {
-    const int jm = j - 1, jp = j + 1;
+  const bool wall = by + 1 == nyb;
+  const int jrow = wall ? ny + 1 : by * nr + r + 1;
+  const bool live = wall ? r == 0 : jrow <= ny;
+  const int j = wall ? ny + 1 : min(jrow, ny), jm = j - 1, jp = j + 1;
+  const double IY1 = met[M_YINT * nyh + j], IY2 = 1.0 - IY1;
+  const double cac = met[M_RDYC * nyh + j];
+  auto wz = [&](int kk) { return (long long)(kk < 0 ? kk + nz : (kk >= nz ? kk - nz : kk)) * g.plane; };
+  if (wall) {
+    // the p interpolations of the few points here come from the caches
+    const int m2 = wrapi(ic - 2, nx), m1 = wrapi(ic - 1, nx), p1 = wrapi(ic + 1, nx);
+    if (own && live)
+      for (int k = k0; k < k1; ++k) {
+        const long long o = (long long)nx * j + (long long)k * g.plane, om = o - nx;
+        const double prloc2 = IY1 * (I1 * pr[om + m2] + I2 * pr[om + m1] + I3 * pr[om + ic] + I4 * pr[om + p1]) +
+                              IY2 * (I1 * pr[o + m2] + I2 * pr[o + m1] + I3 * pr[o + ic] + I4 * pr[o + p1]);
+        const double dudy = (ux[o + ic] - ux[om + ic]) * cac;
+        const double dwdy = (uz[o + ic] - uz[om + ic]) * cac;
+        sv[26] += prloc2 * (dudy + 0.0);
+        sv[32] += dwdy * dwdy;
+        sv[34] += dudy * dudy;
+      }
+  } else {
     const double cacU = met[M_RDYC * nyh + jp], caj = met[M_RDYP * nyh + j];
     const double ap2c = met[M_AP2C * nyh + j], ac2c = met[M_AC2C * nyh + j], am2c = met[M_AM2C * nyh + j];
     const double ap2p = met[M_AP2P * nyh + j], ac2p = met[M_AC2P * nyh + j], am2p = met[M_AM2P * nyh + j];
-    for (int k = k0; k < k1; ++k)
-      for (int i = threadIdx.x; i < g.nx; i += 256) {
-        const Ngh n(g, i, k);
-        auto U = [&](int di, int jj, int dk) { return n(ux, di, jj, dk); };
-        auto V = [&](int di, int jj, int dk) { return n(uy, di, jj, dk); };
-        auto W = [&](int di, int jj, int dk) { return n(uz, di, jj, dk); };
-        auto Pp = [&](int di, int jj, int dk) { return n(pr, di, jj, dk); };
-        const double uxloc = U(0, j, 0) + ucrf, uyloc = V(0, j, 0), uzloc = W(0, j, 0), prloc = Pp(0, j, 0);
-        const double uxCell = I1 * U(-1, j, 0) + I2 * U(0, j, 0) + I3 * U(1, j, 0) + I4 * U(2, j, 0) + ucrf;
-        const double uyCell = (uyloc + V(0, jp, 0)) * 0.5;
-        const double uy_xc = I1 * V(-2, j, 0) + I2 * V(-1, j, 0) + I3 * V(0, j, 0) + I4 * V(1, j, 0);
-        const double uy_xp = I1 * V(-2, jp, 0) + I2 * V(-1, jp, 0) + I3 * V(0, jp, 0) + I4 * V(1, jp, 0);
-        const double uzCell = I1 * W(0, j, -1) + I2 * W(0, j, 0) + I3 * W(0, j, 1) + I4 * W(0, j, 2);
-        const double prloc2 = IY1 * (I1 * Pp(-2, jm, 0) + I2 * Pp(-1, jm, 0) + I3 * Pp(0, jm, 0) + I4 * Pp(1, jm, 0)) +
-                              IY2 * (I1 * Pp(-2, j, 0) + I2 * Pp(-1, j, 0) + I3 * Pp(0, j, 0) + I4 * Pp(1, j, 0));
-        const double dudx = g.dxc1 * U(-1, j, 0) + g.dxc2 * U(0, j, 0) + g.dxc3 * U(1, j, 0) + g.dxc4 * U(2, j, 0);
-        const double dudy = (U(0, j, 0) - U(0, jm, 0)) * cac;
-        const double dudz = g.dzc1 * U(0, j, -2) + g.dzc2 * U(0, j, -1) + g.dzc3 * U(0, j, 0) + g.dzc4 * U(0, j, 1);
-        const double dvdx = g.dxc1 * V(-2, j, 0) + g.dxc2 * V(-1, j, 0) + g.dxc3 * V(0, j, 0) + g.dxc4 * V(1, j, 0);
-        const double dvdy = (V(0, jp, 0) - uyloc) * caj;
-        const double dvdz = g.dzc1 * V(0, j, -2) + g.dzc2 * V(0, j, -1) + g.dzc3 * V(0, j, 0) + g.dzc4 * V(0, j, 1);
-        const double dwdx = g.dxc1 * W(-2, j, 0) + g.dxc2 * W(-1, j, 0) + g.dxc3 * W(0, j, 0) + g.dxc4 * W(1, j, 0);
-        const double dwdy = (uzloc - W(0, jm, 0)) * cac;
-        const double dwdz = g.dzc1 * W(0, j, -1) + g.dzc2 * W(0, j, 0) + g.dzc3 * W(0, j, 1) + g.dzc4 * W(0, j, 2);
-        auto dxx = [&](auto F) {
-          return g.dxxc1 * F(-2, j, 0) + g.dxxc2 * F(-1, j, 0) + g.dxxc3 * F(0, j, 0) + g.dxxc4 * F(1, j, 0) +
-                 g.dxxc5 * F(2, j, 0);
-        };
-        auto dzz = [&](auto F) {
-          return g.dzzc1 * F(0, j, -2) + g.dzzc2 * F(0, j, -1) + g.dzzc3 * F(0, j, 0) + g.dzzc4 * F(0, j, 1) +
-                 g.dzzc5 * F(0, j, 2);
-        };
-        const double dudxx = dxx(U), dudzz = dzz(U);
-        const double dudyy = ap2c * U(0, jp, 0) + ac2c * U(0, j, 0) + am2c * U(0, jm, 0);
-        const double dvdxx = dxx(V), dvdzz = dzz(V);
-        const double dvdyy = ap2p * V(0, jp, 0) + ac2p * V(0, j, 0) + am2p * V(0, jm, 0);
-        const double dwdxx = dxx(W), dwdzz = dzz(W);
-        const double dwdyy = ap2c * W(0, jp, 0) + ac2c * W(0, j, 0) + am2c * W(0, jm, 0);
-        const double vor_x = dwdy - dvdz, vor_y = dudz - dwdx, vor_z = dvdx - dudy;
-        const double dudxC = (-U(2, j, 0) + 8.0 * U(1, j, 0) - 8.0 * U(-1, j, 0) + U(-2, j, 0)) * rdxt;
-        const double dvdxU = g.dxc1 * V(-2, jp, 0) + g.dxc2 * V(-1, jp, 0) + g.dxc3 * V(0, jp, 0) + g.dxc4 * V(1, jp, 0);
-        const double dudyU = (U(0, jp, 0) - U(0, j, 0)) * cacU;
-        const double dudzC = (IY1 * (-U(0, jm, 2) + 8.0 * U(0, jm, 1) - 8.0 * U(0, jm, -1) + U(0, jm, -2)) +
-                              IY2 * (-U(0, j, 2) + 8.0 * U(0, j, 1) - 8.0 * U(0, j, -1) + U(0, j, -2))) *
-                             rdzt;
-        auto c4z = [&](int di) { return -V(di, j, 2) + 8.0 * V(di, j, 1) - 8.0 * V(di, j, -1) + V(di, j, -2); };
-        const double dvdzC = (c4z(-2) * I1 + c4z(-1) * I2 + c4z(0) * I3 + c4z(1) * I4) * rdzt;
+    // LDS slots of the x neighbours i-2..i+2 (clamped for halo threads, whose
+    // sums are dropped)
+    int nb[5];
+#pragma unroll
+    for (int s = 0; s < 5; ++s) {
+      int q = (seg ? i : ic) + s - 2;
+      if (seg) q = q < 0 ? 0 : (q >= lw ? lw - 1 : q);
+      else q = wrapi(q, nx);
+      nb[s] = q;
+    }
+    // a wave-uniform plane and 32-bit byte offsets of the rows j, j-1, j+1
+    const unsigned oj = 8u * (unsigned)(ic + nx * j), om = oj - 8u * nx, op = oj + 8u * nx;
+    const int pbytes = (int)(8 * g.plane);
+    auto ld = [&](const double *a, long long kp, unsigned o) { return bld(plane_rsrc(a + kp, pbytes), o); };
+    double wu[5], wum[5], wv[5], ww[5];
+#pragma unroll
+    for (int s = 0; s < 5; ++s) {
+      const long long kp = wz(k0 + s - 2);
+      wu[s] = ld(ux, kp, oj);
+      wum[s] = ld(ux, kp, om);
+      wv[s] = ld(uy, kp, oj);
+      ww[s] = ld(uz, kp, oj);
+    }
+    struct Plane {
+      double up, vm, vp, wm, wp, p, pm, s;
+    };
+    auto load = [&](int k) {
+      const long long kp = (long long)k * g.plane;
+      Plane q;
+      q.up = ld(ux, kp, op);
+      q.vm = ld(uy, kp, om);
+      q.vp = ld(uy, kp, op);
+      q.wm = ld(uz, kp, om);
+      q.wp = ld(uz, kp, op);
+      q.p = ld(pr, kp, oj);
+      q.pm = ld(pr, kp, om);
+      q.s = SC ? ld(sc, kp, oj) : 0.0;
+      return q;
+    };
+    Plane cur = load(k0);
+    for (int k = k0; k < k1; ++k) {
+      double *X = xr + (size_t)((k & 1) * nr + r) * T_NROWS * lw;
+      const double c4own = -wv[4] + 8.0 * wv[3] - 8.0 * wv[1] + wv[0];
+      if (in) {
+        X[T_U * lw + i] = wu[2];
+        X[T_V * lw + i] = wv[2];
+        X[T_VP * lw + i] = cur.vp;
+        X[T_W * lw + i] = ww[2];
+        X[T_P * lw + i] = cur.p;
+        X[T_PM * lw + i] = cur.pm;
+        X[T_C4 * lw + i] = c4own;
+      }
+      // the next plane's values, in flight while this one is formed (the last
+      // plane reloads its own)
+      const Plane nxt = load(k + 1 < k1 ? k + 1 : k);
+      const long long kn = wz(k + 3);
+      const double nu = ld(ux, kn, oj), num = ld(ux, kn, om), nv = ld(uy, kn, oj), nw = ld(uz, kn, oj);
+      __syncthreads();
+      auto at = [&](int row, int d) { return X[row * lw + nb[d + 2]]; };
+      const double u0 = wu[2], uyloc = wv[2], uzloc = ww[2], prloc = cur.p;
+      const double u_m2 = at(T_U, -2), u_m1 = at(T_U, -1), u_p1 = at(T_U, 1), u_p2 = at(T_U, 2);
+      const double v_m2 = at(T_V, -2), v_m1 = at(T_V, -1), v_p1 = at(T_V, 1), v_p2 = at(T_V, 2);
+      const double y_m2 = at(T_VP, -2), y_m1 = at(T_VP, -1), y_p1 = at(T_VP, 1);
+      const double w_m2 = at(T_W, -2), w_m1 = at(T_W, -1), w_p1 = at(T_W, 1), w_p2 = at(T_W, 2);
+      const double uxloc = u0 + ucrf;
+      const double uxCell = I1 * u_m1 + I2 * u0 + I3 * u_p1 + I4 * u_p2 + ucrf;
+      const double uyCell = (uyloc + cur.vp) * 0.5;
+      const double uy_xc = I1 * v_m2 + I2 * v_m1 + I3 * uyloc + I4 * v_p1;
+      const double uy_xp = I1 * y_m2 + I2 * y_m1 + I3 * cur.vp + I4 * y_p1;
+      const double uzCell = I1 * ww[1] + I2 * ww[2] + I3 * ww[3] + I4 * ww[4];
+      const double prloc2 =
+          IY1 * (I1 * at(T_PM, -2) + I2 * at(T_PM, -1) + I3 * cur.pm + I4 * at(T_PM, 1)) +
+          IY2 * (I1 * at(T_P, -2) + I2 * at(T_P, -1) + I3 * prloc + I4 * at(T_P, 1));
+      const double dudx = g.dxc1 * u_m1 + g.dxc2 * u0 + g.dxc3 * u_p1 + g.dxc4 * u_p2;
+      const double dudy = (u0 - wum[2]) * cac;
+      const double dudz = g.dzc1 * wu[0] + g.dzc2 * wu[1] + g.dzc3 * wu[2] + g.dzc4 * wu[3];
+      const double dvdx = g.dxc1 * v_m2 + g.dxc2 * v_m1 + g.dxc3 * uyloc + g.dxc4 * v_p1;
+      const double dvdy = (cur.vp - uyloc) * caj;
+      const double dvdz = g.dzc1 * wv[0] + g.dzc2 * wv[1] + g.dzc3 * wv[2] + g.dzc4 * wv[3];
+      const double dwdx = g.dxc1 * w_m2 + g.dxc2 * w_m1 + g.dxc3 * uzloc + g.dxc4 * w_p1;
+      const double dwdy = (uzloc - cur.wm) * cac;
+      const double dwdz = g.dzc1 * ww[1] + g.dzc2 * ww[2] + g.dzc3 * ww[3] + g.dzc4 * ww[4];
+      auto dxx = [&](double a, double b, double c, double d, double e) {
+        return g.dxxc1 * a + g.dxxc2 * b + g.dxxc3 * c + g.dxxc4 * d + g.dxxc5 * e;
+      };
+      auto dzz = [&](const double (&w)[5]) {
+        return g.dzzc1 * w[0] + g.dzzc2 * w[1] + g.dzzc3 * w[2] + g.dzzc4 * w[3] + g.dzzc5 * w[4];
+      };
+      const double dudxx = dxx(u_m2, u_m1, u0, u_p1, u_p2), dudzz = dzz(wu);
+      const double dudyy = ap2c * cur.up + ac2c * u0 + am2c * wum[2];
+      const double dvdxx = dxx(v_m2, v_m1, uyloc, v_p1, v_p2), dvdzz = dzz(wv);
+      const double dvdyy = ap2p * cur.vp + ac2p * uyloc + am2p * cur.vm;
+      const double dwdxx = dxx(w_m2, w_m1, uzloc, w_p1, w_p2), dwdzz = dzz(ww);
+      const double dwdyy = ap2c * cur.wp + ac2c * uzloc + am2c * cur.wm;
+      const double vor_x = dwdy - dvdz, vor_y = dudz - dwdx, vor_z = dvdx - dudy;
+      const double dudxC = (-u_p2 + 8.0 * u_p1 - 8.0 * u_m1 + u_m2) * rdxt;
+      const double dvdxU = g.dxc1 * y_m2 + g.dxc2 * y_m1 + g.dxc3 * cur.vp + g.dxc4 * y_p1;
+      const double dudyU = (cur.up - u0) * cacU;
+      const double dudzC = (IY1 * (-wum[4] + 8.0 * wum[3] - 8.0 * wum[1] + wum[0]) +
+                            IY2 * (-wu[4] + 8.0 * wu[3] - 8.0 * wu[1] + wu[0])) *
+                           rdzt;
+      const double dvdzC = (at(T_C4, -2) * I1 + at(T_C4, -1) * I2 + c4own * I3 + at(T_C4, 1) * I4) * rdzt;
+      if (own && live) {
         sv[0] += uxloc;
         sv[1] += uyloc;
         sv[2] += uzloc;
@@ -1562,7 +1682,7 @@ __global__ void __launch_bounds__(256) k_stat_partial(Geo g, double ucrf, const 
         sv[33] += vor_y * vor_y;
         sv[34] += vor_z * vor_z;
         if constexpr (SC) {
-          const double scloc = n(sc, 0, j, 0);
+          const double scloc = cur.s;
           sv[35] += scloc;
           sv[36] += scloc * scloc;
           sv[37] += scloc * uxCell;
@@ -1570,43 +1690,50 @@ __global__ void __launch_bounds__(256) k_stat_partial(Geo g, double ucrf, const 
           sv[39] += scloc * uzCell;
         }
       }
-  } else {
-    const int jm = j - 1;
-    for (int k = k0; k < k1; ++k)
-      for (int i = threadIdx.x; i < g.nx; i += 256) {
-        const Ngh n(g, i, k);
-        auto Pp = [&](int di, int jj) { return n(pr, di, jj, 0); };
-        const double prloc2 = IY1 * (I1 * Pp(-2, jm) + I2 * Pp(-1, jm) + I3 * Pp(0, jm) + I4 * Pp(1, jm)) +
-                              IY2 * (I1 * Pp(-2, j) + I2 * Pp(-1, j) + I3 * Pp(0, j) + I4 * Pp(1, j));
-        const double dudy = (n(ux, 0, j, 0) - n(ux, 0, jm, 0)) * cac;
-        const double dwdy = (n(uz, 0, j, 0) - n(uz, 0, jm, 0)) * cac;
-        sv[26] += prloc2 * (dudy + 0.0);
-        sv[32] += dwdy * dwdy;
-        sv[34] += dudy * dudy;
-      }
-  }
-  double *out = part + ((long long)blockIdx.y * gridDim.x + blockIdx.x) * NS;
+      cur = nxt;
 #pragma unroll
-  for (int q = 0; q < NS; ++q) {
-    const double s = block_sum(sv[q], sh);
-    if (threadIdx.x == 0) out[q] = s;
-    __syncthreads();
+      for (int s = 0; s < 4; ++s) {
+        wu[s] = wu[s + 1];
+        wum[s] = wum[s + 1];
+        wv[s] = wv[s + 1];
+        ww[s] = ww[s + 1];
+      }
+      wu[4] = nu;
+      wum[4] = num;
+      wv[4] = nv;
+      ww[4] = nw;
+    }
+  }
+  // a wavefront lies in one row (blockDim.x is a multiple of 64): its sums, then
+  // those of the row's wavefronts in order
+  const int t = r * (int)blockDim.x + i, wv_id = t >> 6, wpr = (int)blockDim.x >> 6;
+  int idx;
+  wave_sums<NS>(sv, t & 63, &idx);
+  if (idx >= 0) wsum[wv_id][idx] = sv[0];
+  __syncthreads();
+  for (int q = t; q < nr * NS; q += (int)(blockDim.x * blockDim.y)) {
+    const int rr = q / NS, e = q - rr * NS;
+    const int row = wall ? ny + 1 : by * nr + rr + 1;
+    if ((wall && rr > 0) || row > ny + (wall ? 1 : 0)) continue;
+    double s = 0.0;
+    for (int w = 0; w < wpr; ++w) s += wsum[rr * wpr + w][e];
+    part[((long long)(row - 1) * nparts + pt) * NS + e] = s;
   }
 }
 
-// SumStat(q, j) += inxz * (sum over chunks in order); one thread per (q, j)
+// SumStat(q, j) += inxz * (sum over chunks in order); one thread per (q, j).
+// PrGradsum += PrGradAver (:416) with it.
 __global__ void __launch_bounds__(256) k_stat_final(const double *__restrict__ part, int nchunk, int ns, int nyp,
-                                                    double inxz, double *__restrict__ sumstat) {
+                                                    double inxz, double *__restrict__ sumstat,
+                                                    double *__restrict__ scal) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t == 0) scal[S_PRGSUM] += scal[S_PRGRAD];
   if (t >= ns * nyp) return;
   const int q = t % ns, j = t / ns;
   double s = 0.0;
   for (int c = 0; c < nchunk; ++c) s += part[((long long)j * nchunk + c) * ns + q];
   sumstat[t] += s * inxz;
 }
-
-// PrGradsum += PrGradAver (:416), on the device
-__global__ void k_stat_prgrad(double *scal) { scal[S_PRGSUM] += scal[S_PRGRAD]; }
 
 int launch_stat(ptc_ctx *c, const double *ux, const double *uy, const double *uz, const double *pr,
                 const double *sc) {
@@ -1615,24 +1742,31 @@ int launch_stat(ptc_ctx *c, const double *ux, const double *uy, const double *uz
     PTC_HIP(hipMalloc(&c->d_stat, sizeof(double) * (size_t)ns * nyp));
     PTC_TRY(fill_device(c, c->d_stat, (long long)ns * nyp, 0.0));
   }
-  // chunks of k planes: ~8 blocks per CU over all planes
-  const int want = std::max(1, (c->n_cu * 8) / nyp);
-  const int nchunk = std::min(c->nz, want);
-  const int kc = (c->nz + nchunk - 1) / nchunk;
-  const int nblk = (c->nz + kc - 1) / kc;
+  // rows: whole up to 256 points, else segments of 252 with a two-column halo;
+  // short rows share a workgroup of 256 threads
+  const int tx = c->nx <= 256 ? (c->nx + 63) / 64 * 64 : 256, seg = c->nx <= 256 ? 0 : tx - 4;
+  const int ty = 256 / tx, lw = seg ? tx : c->nx, nseg = seg ? (c->nx + seg - 1) / seg : 1;
+  const int nyb = (c->ny + ty - 1) / ty;
+  // chunks of k planes: four rounds of the two workgroups per CU, at least 8
+  // planes each (a chunk loads a window of four planes more)
+  const long long tiles = (long long)nyb * nseg;
+  const int want = (int)std::max<long long>(1, (8LL * c->n_cu + tiles - 1) / tiles);
+  const int nchunk = std::max(1, std::min(want, c->nz / 8));
+  const int kc = (c->nz + nchunk - 1) / nchunk, nch = (c->nz + kc - 1) / kc;
+  const int nblk = nseg * nch;
   PTC_TRY(ensure_red(c, nblk * nyp * ns));
+  const dim3 grid((unsigned)nblk, (unsigned)(nyb + 1)), blk((unsigned)tx, (unsigned)ty);
+  const size_t lds = sizeof(double) * 2 * T_NROWS * (size_t)lw * ty;
   if (c->prm.scalar)
-    hipLaunchKernelGGL(k_stat_partial<true>, dim3(nblk, nyp), dim3(256), 0, c->stream, c->geo, c->prm.ucrf, ux, uy,
-                       uz, pr, sc, kc, c->d_red);
+    hipLaunchKernelGGL(k_stat_rows<true>, grid, blk, lds, c->stream, c->geo, c->prm.ucrf, ux, uy, uz, pr, sc, kc, nch,
+                       seg, lw, kVelXcdRun, c->d_red);
   else
-    hipLaunchKernelGGL(k_stat_partial<false>, dim3(nblk, nyp), dim3(256), 0, c->stream, c->geo, c->prm.ucrf, ux, uy,
-                       uz, pr, sc, kc, c->d_red);
+    hipLaunchKernelGGL(k_stat_rows<false>, grid, blk, lds, c->stream, c->geo, c->prm.ucrf, ux, uy, uz, pr, sc, kc, nch,
+                       seg, lw, kVelXcdRun, c->d_red);
   PTC_HIP(hipGetLastError());
   const double inxz = 1.0 / ((double)c->nx * (double)c->nz);
   hipLaunchKernelGGL(k_stat_final, dim3((ns * nyp + 255) / 256), dim3(256), 0, c->stream, c->d_red, nblk, ns, nyp,
-                     inxz, c->d_stat);
-  PTC_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_stat_prgrad, dim3(1), dim3(1), 0, c->stream, c->d_scal);
+                     inxz, c->d_stat, c->d_scal);
   PTC_HIP(hipGetLastError());
   ++c->nfstime;
   return PTC_OK;
