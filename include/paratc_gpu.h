@@ -219,13 +219,15 @@ int ptc_poisson_set(ptc_ctx *ctx, int knob, int value);
  * 3 both); 0 where the knob's variant is not in use) */
 int ptc_poisson_get_knob(ptc_ctx *ctx, int knob, int *value);
 /* Workgroup shape of the row-marching clcRhsXYZ kernel (0 = automatic):
- *   PTC_RHS_SEGMENT_THREADS  threads per row segment where rows are longer
- *                            than 512 points: 64, 128 or 256 (automatic 128)
+ *   PTC_RHS_SEGMENT_THREADS  threads per row segment where rows go in
+ *                            segments (longer than 128 points, except 245 to
+ *                            256 and, on small grids, 257 to 512): 64, 128 or
+ *                            256 (automatic 128)
  *   PTC_RHS_ROWS             rows j per workgroup, at most 512 threads in
  *                            all: the inner rows' j-1 / j+1 values come
- *                            through LDS (automatic: 4 for rows in
- *                            segments, 2 where a whole row is at most 128
- *                            threads, else 1)
+ *                            through LDS (automatic: 4 for rows of at most 64
+ *                            points, 2 up to 512 points, 2 or 4 for longer
+ *                            rows by the size of a field)
  *   PTC_RHS_XCD_RUN          consecutive tiles run on one XCD (1 = plain
  *                            order; automatic 32)
  *   PTC_RHS_MIN_PLANES       z planes per chunk at least (each chunk starts

@@ -99,25 +99,37 @@ __device__ __forceinline__ double block_max(double v, double *sh) {
 // and kept in short queues.  Operand order follows the reference's
 // expressions except that those products are formed before their difference
 // weight is applied.
+//
+// The LDS rows of a quantity are the workgroup's rows with one ghost row below
+// and one above: the first and the last row's threads also load the row outside,
+// so every thread reads its j-1 and j+1 values from the rows beside its own and
+// the loop has no branch around a global access.  The
+// loads of plane k+1 are issued at the top of plane k into registers of their
+// own and waited for at its end, before plane k's stores, so a plane's latency
+// is hidden by the arithmetic: with the loads at the end (needed at the top of
+// the next plane, behind the stores) the wavefronts of a workgroup idled
+// together on every plane.  128x96x128: 51.0 -> 42 us (104 B per point at 3.9
+// TB/s, two wavefronts per SIMD at 218 VGPRs); 256x128x192 with the scalar 243
+// -> 215 us; 4608x140x700 15.6 -> 15.3 ms, where the counted traffic (158 B per
+// point) already moves at 4.7 TB/s, near the copy rate.
 enum {
-  X_UX = 0,  // ux(., j, k)
-  X_UY,      // uy(., j, k)
-  X_UZ,      // uz(., j, k)
+  X_UX = 0,  // ux(., j, k); ghost rows both sides
+  X_UY,      // uy(., j, k); both sides
+  X_UZ,      // uz(., j, k); above
   X_UZ2,     // uz(., j, k + 2)
-  X_P,       // p(., j, k)
-  X_UXM,     // ux(., j - 1, k)
-  X_UYP,     // uy(., j + 1, k)
+  X_P,       // p(., j, k); below
   X_R,       // uzhx * (uxhz + ucrf) at (., j, k)
-  X_SC,      // scalar(., j, k)
-  X_UYF,     // uy(., j, k + 2): the next window entry of row j - 1's uy(j + 1) window
-  X_UZF,     // uz(., j, k + 3): the next window entry of row j + 1's uz(j - 1) window
+  X_SC,      // scalar(., j, k); both sides
+  X_UYF,     // uy(., j, k + 2): the next window entry of row j - 1's uy(j + 1) window; above
+  X_UZF,     // uz(., j, k + 3): the next window entry of row j + 1's uz(j - 1) window; below
   X_NROWS
 };
 
 // Raw buffer access to one plane: the plane's base address and size live in
 // scalar registers and a lane adds a 32-bit byte offset, so a load costs one
 // VGPR for the address whatever the number of fields in flight.  Offsets past
-// the plane read zero and drop stores (the row kernels never form them).
+// the plane read zero without touching memory and drop stores: kNoAccess turns an
+// access off without a branch.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const double *base, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(base), (short)0, bytes, 0x00020000);
 }
@@ -129,7 +141,10 @@ __device__ __forceinline__ void bst(__amdgpu_buffer_rsrc_t r, unsigned off, doub
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V2, v), r, off, 0, 0);
 }
 
-template <bool SC, int MAXT>
+constexpr unsigned kNoAccess = 0xFFFFFFF0u;
+
+// ONE: one row per workgroup (its threads load both ghost rows)
+template <bool SC, int MAXT, bool ONE>
 __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, const double *__restrict__ ux,
                                                   const double *__restrict__ uy, const double *__restrict__ uz,
                                                   const double *__restrict__ sc, const double *__restrict__ p,
@@ -138,7 +153,7 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
                                                   double *__restrict__ hx, double *__restrict__ hy,
                                                   double *__restrict__ hz, double *__restrict__ hc,
                                                   double *__restrict__ s3part, int seg, int lw, int grp) {
-  extern __shared__ double xr[];  // X_NROWS x (rows of the workgroup) rows of lw values
+  extern __shared__ double xr[];  // X_NROWS x (rows of the workgroup + 2 ghosts) rows of lw values
   const int nx = g.nx, nz = g.nz;
   const int i = threadIdx.x;
   // tile (segment bx, row group by, z chunk bz): runs of grp consecutive tiles,
@@ -161,11 +176,11 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
   const int ic = seg ? gcol : (i < nx ? i : 0);
   const int j = vrow ? jrow : g.ny, jp = j + 1;
   const int nyp = g.ny + 1;
-  // the j-1 and j+1 rows of a row inside the workgroup are its neighbours'
-  // rows: their values come through LDS, and only the workgroup's edge rows
-  // load them from HBM
-  const bool lo_lds = r > 0;
-  const bool hi_lds = r + 1 < nr && jrow + 1 <= g.ny;
+  // ghost duties: the first row's threads load the row below, the last row's
+  // (a mirror row or not) the row above the last valid one
+  const bool dlo = r == 0, dhi = r == nr - 1;
+  const int jlo = by * nr, jlast = min(by * nr + nr, g.ny), jhi = jlast + 1;
+  const int hslot = jlast - by * nr + 1;
   const int k0 = bz * kc, k1 = min(k0 + kc, nz);
   const long long pl = g.plane;
   const double *M = g.met;
@@ -202,14 +217,12 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
     else q = q < 0 ? q + nx : (q >= nx ? q - nx : q);
     nb[s] = q;
   }
-  // LDS row of quantity `row` for workgroup row rr
-  auto LR = [&](int row, int rr) { return (row * nr + rr) * lw; };
-  auto X = [&](int row, int d) { return xr[LR(row, r) + nb[d + 3]]; };
-  // ux(j-1) and uy(j+1) with their x neighbours: the neighbouring rows' ux and
-  // uy rows inside the workgroup, else this row's own copies
-  const int uxm_row = lo_lds ? LR(X_UX, r - 1) : LR(X_UXM, r), uyp_row = hi_lds ? LR(X_UY, r + 1) : LR(X_UYP, r);
-  auto XUXM = [&](int d) { return xr[uxm_row + nb[d + 3]]; };
-  auto XUYP = [&](int d) { return xr[uyp_row + nb[d + 3]]; };
+  // LDS row of quantity `row` in slot q: the workgroup's row q - 1, ghosts at 0
+  // and past its last valid row
+  auto LR = [&](int row, int q) { return (row * (nr + 2) + q) * lw; };
+  auto X = [&](int row, int d) { return xr[LR(row, r + 1) + nb[d + 3]]; };
+  auto XM = [&](int row, int d) { return xr[LR(row, r) + nb[d + 3]]; };      // row j - 1
+  auto XP = [&](int row, int d) { return xr[LR(row, r + 2) + nb[d + 3]]; };  // row j + 1
   auto wz = [&](int kk) { return kk < 0 ? kk + nz : (kk >= nz ? kk - nz : kk); };
   auto at = [&](int kk) { return (long long)wz(kk) * pl; };
   // byte offsets of this column at rows j, j-1, j+1 inside a plane: loads and
@@ -219,7 +232,6 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
   auto ldp = [&](const double *a, int kk, unsigned off) { return bld(plane_rsrc(a + at(kk), pbytes), off); };
 
   double wux[7], wuy[7], wuz[7], wsc[7], wp[4], wuyp[4], wuzm[4];
-  double ux_m, ux_p, uy_m, uz_p, p_m, sc_m = 0.0, sc_p = 0.0;
 #pragma unroll
   for (int s = 0; s < 7; ++s) {
     wux[s] = ldp(ux, k0 + s - 3, bj);
@@ -233,17 +245,24 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
     wuyp[s] = ldp(uy, k0 + s - 2, bjp);
     wuzm[s] = ldp(uz, k0 + s - 1, bjm);
   }
-  {
-    ux_m = ldp(ux, k0, bjm);
-    ux_p = ldp(ux, k0, bjp);
-    uy_m = ldp(uy, k0, bjm);
-    uz_p = ldp(uz, k0, bjp);
-    p_m = ldp(p, k0, bjm);
-    if (SC) {
-      sc_m = ldp(sc, k0, bjm);
-      sc_p = ldp(sc, k0, bjp);
-    }
-  }
+  // The ghost rows' values of one plane: ux, uy, p (below) or uz (above), the
+  // scalar, and uz three planes ahead (below) or uy two ahead (above).  A thread
+  // with one duty keeps them in lo whichever side it loads.
+  struct Ghost {
+    double x, y, c, s, f;
+  };
+  const unsigned olo = 8u * (unsigned)(ic + nx * jlo), ohi = 8u * (unsigned)(ic + nx * jhi);
+  const unsigned og = ONE || dlo ? olo : (dhi ? ohi : kNoAccess);
+  const double *pc = ONE || dlo ? p : uz, *pf = ONE || dlo ? uz : uy;
+  const int kf = ONE || dlo ? 3 : 2;
+  auto ldg = [&](int k) {
+    return Ghost{ldp(ux, k, og), ldp(uy, k, og), ldp(pc, k, og), SC ? ldp(sc, k, og) : 0.0, ldp(pf, k + kf, og)};
+  };
+  auto ldg_hi = [&](int k) {
+    return Ghost{ldp(ux, k, ohi), ldp(uy, k, ohi), ldp(uz, k, ohi), SC ? ldp(sc, k, ohi) : 0.0, ldp(uy, k + 2, ohi)};
+  };
+  Ghost glo = ldg(k0), ghi{};
+  if (ONE) ghi = ldg_hi(k0);
   // queues: Q(k') = uxhz * uzhx for k' = k-1..k+2, R(k') = uzhx * (uxhz + ucrf)
   // for k' = k..k+2, uzhx from the uz rows of planes k0-1..k0+1 first
   double Q[4], R[3];
@@ -251,9 +270,9 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
     return c1 * wux[s] + c2 * wux[s + 1] + c3 * wux[s + 2] + c4 * wux[s + 3];
   };
   if (lds_in) {
-    xr[LR(0, r) + i] = wuz[2];
-    xr[LR(1, r) + i] = wuz[3];
-    xr[LR(2, r) + i] = wuz[4];
+    xr[LR(0, r + 1) + i] = wuz[2];
+    xr[LR(1, r + 1) + i] = wuz[3];
+    xr[LR(2, r + 1) + i] = wuz[4];
   }
   __syncthreads();
   {
@@ -268,45 +287,53 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
     R[1] = zx[2] * (hz2 + ucrf);
   }
   double s3 = 0.0;
-  // the old right-hand sides of a plane are loaded with the previous plane's
-  // window entries, a plane ahead of their use
   auto ldh = [&](const double *a, int kk) { return bld(plane_rsrc(a + (long long)kk * pl, pbytes), bj); };
-  double hxo = ldh(hx, k0), hyo = ldh(hy, k0), hzo = ldh(hz, k0), hco = SC ? ldh(hc, k0) : 0.0;
+  const unsigned bst_off = act ? bj : kNoAccess;
   for (int k = k0; k < k1; ++k) {
     const long long kp = (long long)k * pl;
+    // this plane's old right-hand sides, then the next plane's window entries
+    // and ghost rows
+    const double hxo = ldh(hx, k), hyo = ldh(hy, k), hzo = ldh(hz, k), hco = SC ? ldh(hc, k) : 0.0;
+    const double nux = ldp(ux, k + 4, bj), nuy = ldp(uy, k + 4, bj), nuz = ldp(uz, k + 4, bj),
+                 nsc = SC ? ldp(sc, k + 4, bj) : 0.0, np = ldp(p, k + 2, bj);
+    const Ghost nlo = ldg(k + 1);
+    Ghost nhi{};
+    if (ONE) nhi = ldg_hi(k + 1);
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();  // the previous plane's reads are done
     if (lds_in) {
-      xr[LR(X_UX, r) + i] = wux[3];
-      xr[LR(X_UY, r) + i] = wuy[3];
-      xr[LR(X_UZ, r) + i] = wuz[3];
-      xr[LR(X_UZ2, r) + i] = wuz[5];
-      xr[LR(X_P, r) + i] = wp[2];
-      if (!lo_lds) xr[LR(X_UXM, r) + i] = ux_m;
-      if (!hi_lds) xr[LR(X_UYP, r) + i] = wuyp[2];
-      xr[LR(X_R, r) + i] = R[0];
-      if (SC) xr[LR(X_SC, r) + i] = wsc[3];
-      if (nr > 1) {
-        xr[LR(X_UYF, r) + i] = wuy[5];
-        xr[LR(X_UZF, r) + i] = wuz[6];
+      if (vrow) {
+        xr[LR(X_UX, r + 1) + i] = wux[3];
+        xr[LR(X_UY, r + 1) + i] = wuy[3];
+        xr[LR(X_UZ, r + 1) + i] = wuz[3];
+        xr[LR(X_UZ2, r + 1) + i] = wuz[5];
+        xr[LR(X_P, r + 1) + i] = wp[2];
+        xr[LR(X_R, r + 1) + i] = R[0];
+        if (SC) xr[LR(X_SC, r + 1) + i] = wsc[3];
+        if (!ONE) {
+          xr[LR(X_UYF, r + 1) + i] = wuy[5];
+          xr[LR(X_UZF, r + 1) + i] = wuz[6];
+        }
+      }
+      if (ONE || dlo || dhi) {
+        const int q = ONE || dlo ? 0 : hslot;
+        xr[LR(X_UX, q) + i] = glo.x;
+        xr[LR(X_UY, q) + i] = glo.y;
+        xr[LR(ONE || dlo ? X_P : X_UZ, q) + i] = glo.c;
+        if (SC) xr[LR(X_SC, q) + i] = glo.s;
+        xr[LR(ONE || dlo ? X_UZF : X_UYF, q) + i] = glo.f;
+      }
+      if (ONE) {
+        xr[LR(X_UX, 2) + i] = ghi.x;
+        xr[LR(X_UY, 2) + i] = ghi.y;
+        xr[LR(X_UZ, 2) + i] = ghi.c;
+        if (SC) xr[LR(X_SC, 2) + i] = ghi.s;
+        xr[LR(X_UYF, 2) + i] = ghi.f;
       }
     }
     __syncthreads();
-    // this plane's j-1 / j+1 values of the rows inside the workgroup, and the
-    // next entries of the uy(j+1) and uz(j-1) windows
-    double nwuyp = 0.0, nwuzm = 0.0;
-    if (lo_lds) {
-      ux_m = xr[LR(X_UX, r - 1) + nb[3]];
-      uy_m = xr[LR(X_UY, r - 1) + nb[3]];
-      p_m = xr[LR(X_P, r - 1) + nb[3]];
-      if (SC) sc_m = xr[LR(X_SC, r - 1) + nb[3]];
-      nwuzm = xr[LR(X_UZF, r - 1) + nb[3]];
-    }
-    if (hi_lds) {
-      ux_p = xr[LR(X_UX, r + 1) + nb[3]];
-      uz_p = xr[LR(X_UZ, r + 1) + nb[3]];
-      if (SC) sc_p = xr[LR(X_SC, r + 1) + nb[3]];
-      nwuyp = xr[LR(X_UYF, r + 1) + nb[3]];
-    }
+    const double ux_m = XM(X_UX, 0), uy_m = XM(X_UY, 0), p_m = XM(X_P, 0), sc_m = SC ? XM(X_SC, 0) : 0.0;
+    const double ux_p = XP(X_UX, 0), uz_p = XP(X_UZ, 0), sc_p = SC ? XP(X_SC, 0) : 0.0;
     // the products two planes ahead
     {
       const double zx2 = c1 * X(X_UZ2, -2) + c2 * X(X_UZ2, -1) + c3 * X(X_UZ2, 0) + c4 * X(X_UZ2, 1);
@@ -334,7 +361,7 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
       const double h11 = ex1 * a0 * (a0 + ucrf) + ex2 * a1 * (a1 + ucrf) + (-ex2) * a2 * (a2 + ucrf) +
                          (-ex1) * a3 * (a3 + ucrf);
       const double uyhx_p =
-          top ? 0.0 : c1 * XUYP(-2) + c2 * XUYP(-1) + c3 * wuyp[2] + c4 * XUYP(1);
+          top ? 0.0 : c1 * XP(X_UY, -2) + c2 * XP(X_UY, -1) + c3 * wuyp[2] + c4 * XP(X_UY, 1);
       const double uyhx_c = c1 * xy[1] + c2 * xy[2] + c3 * xy[3] + c4 * xy[4];
       const double h12 = (uyhx_p * uxhyp - uyhx_c * uxhyc) * rdyp;
       const double h13 = ez1 * Q[0] + ez2 * Q[1] + (-ez2) * Q[2] + (-ez1) * Q[3];
@@ -357,10 +384,10 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
     double ry, cy;
     {
       const double qs = 0.25 * rdyc;
-      const double uxhym = IY1 * XUXM(-1) + IY2 * xu[2] + ucrf;
+      const double uxhym = IY1 * XM(X_UX, -1) + IY2 * xu[2] + ucrf;
       const double uxhyc = IY1 * ux_m + IY2 * xu[3] + ucrf;
-      const double uxhyp = IY1 * XUXM(1) + IY2 * xu[4] + ucrf;
-      const double uxhyu = IY1 * XUXM(2) + IY2 * xu[5] + ucrf;
+      const double uxhyp = IY1 * XM(X_UX, 1) + IY2 * xu[4] + ucrf;
+      const double uxhyu = IY1 * XM(X_UX, 2) + IY2 * xu[5] + ucrf;
       const double uzhym = IY1 * wuzm[0] + IY2 * wuz[2];
       const double uzhyc = IY1 * wuzm[1] + IY2 * wuz[3];
       const double uzhyp = IY1 * wuzm[2] + IY2 * wuz[4];
@@ -450,20 +477,10 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
       rc = cf.gamma * cc + cf.theta * hco + 2.0 * cf.beta_sc * d22;
     }
 
-    if (act) {
-      bst(plane_rsrc(rhsx + kp, pbytes), bj, rx);
-      bst(plane_rsrc(rhsy + kp, pbytes), bj, ry);
-      bst(plane_rsrc(rhsz + kp, pbytes), bj, rz);
-      bst(plane_rsrc(hx + kp, pbytes), bj, cx);
-      bst(plane_rsrc(hy + kp, pbytes), bj, cy);
-      bst(plane_rsrc(hz + kp, pbytes), bj, cz);
-      if (SC) {
-        bst(plane_rsrc(rhsc + kp, pbytes), bj, rc);
-        bst(plane_rsrc(hc + kp, pbytes), bj, cc);
-      }
-    }
-
-    // advance one plane: shift the windows and queues, load the new entries
+    // advance one plane: the next entries of the uy(j+1) and uz(j-1) windows
+    // are the neighbour rows'; the other windows and the ghosts take the loads
+    // of the top, waited for before the stores are issued
+    const double nwuzm = XM(X_UZF, 0), nwuyp = XP(X_UYF, 0);
 #pragma unroll
     for (int s = 0; s < 6; ++s) {
       wux[s] = wux[s + 1];
@@ -480,36 +497,25 @@ __global__ void __launch_bounds__(MAXT) k_rhs_rows(Geo g, RhsCoef cf, int kc, co
     }
     R[0] = R[1];
     R[1] = R[2];
-    {
-      wux[6] = ldp(ux, k + 4, bj);
-      wuy[6] = ldp(uy, k + 4, bj);
-      wuz[6] = ldp(uz, k + 4, bj);
-      if (SC) wsc[6] = ldp(sc, k + 4, bj);
-      wp[3] = ldp(p, k + 2, bj);
-      // the edge rows load their outside neighbour row; the others take it
-      // from LDS in the next plane
-      if (lo_lds) {
-        wuzm[3] = nwuzm;
-      } else {
-        wuzm[3] = ldp(uz, k + 3, bjm);
-        ux_m = ldp(ux, k + 1, bjm);
-        uy_m = ldp(uy, k + 1, bjm);
-        p_m = ldp(p, k + 1, bjm);
-        if (SC) sc_m = ldp(sc, k + 1, bjm);
-      }
-      if (hi_lds) {
-        wuyp[3] = nwuyp;
-      } else {
-        wuyp[3] = ldp(uy, k + 2, bjp);
-        ux_p = ldp(ux, k + 1, bjp);
-        uz_p = ldp(uz, k + 1, bjp);
-        if (SC) sc_p = ldp(sc, k + 1, bjp);
-      }
-      const int kn = k + 1 < k1 ? k + 1 : k;  // the last plane reloads its own
-      hxo = ldh(hx, kn);
-      hyo = ldh(hy, kn);
-      hzo = ldh(hz, kn);
-      if (SC) hco = ldh(hc, kn);
+    wux[6] = nux;
+    wuy[6] = nuy;
+    wuz[6] = nuz;
+    if (SC) wsc[6] = nsc;
+    wp[3] = np;
+    wuzm[3] = nwuzm;
+    wuyp[3] = nwuyp;
+    glo = nlo;
+    if (ONE) ghi = nhi;
+    __builtin_amdgcn_sched_barrier(0);
+    bst(plane_rsrc(rhsx + kp, pbytes), bst_off, rx);
+    bst(plane_rsrc(rhsy + kp, pbytes), bst_off, ry);
+    bst(plane_rsrc(rhsz + kp, pbytes), bst_off, rz);
+    bst(plane_rsrc(hx + kp, pbytes), bst_off, cx);
+    bst(plane_rsrc(hy + kp, pbytes), bst_off, cy);
+    bst(plane_rsrc(hz + kp, pbytes), bst_off, cz);
+    if (SC) {
+      bst(plane_rsrc(rhsc + kp, pbytes), bst_off, rc);
+      bst(plane_rsrc(hc + kp, pbytes), bst_off, cc);
     }
   }
   if (cf.s3_mode) {
@@ -1024,25 +1030,35 @@ static int pt_nblocks(const ptc_ctx *c) {
   return (int)(gr.x * gr.y * gr.z);
 }
 
-// row-marching RHS: one workgroup per (row segment, group of rows j, k
-// chunk).  Rows of at most 512 points are one segment (a 1024-thread
-// workgroup would spill); longer rows go in segments of tx - 6 columns with a
-// 3-column halo either side.  A workgroup of ty rows takes the j-1 and j+1
-// rows of its inner rows from LDS, so only its edge rows read a neighbour row
-// from HBM: at 4608x140x700 (SC) 128-thread segments of two rows ran 16.4-16.7
-// ms against 17.2 ms for one row of 256 threads, and four rows of 64 threads
-// 16.3 ms (the halo columns cost what the edge rows save); 512-thread
-// workgroups of two rows of 256 ran 17.3 ms, of four rows of 128 (one per
-// CU, half the edge rows of two) 15.7 against 16.1 ms for two rows of 128.  The k chunks
-// are many enough for about 96 wavefronts per CU over the launch (more rounds
-// of resident workgroups, so the partial last one costs less: the RHS alone
-// 15.3 against 15.4 ms at 4608x140x700 and 3.01 against 3.07 ms at 1536 x 192
-// x 256 with 48) and at least 16 planes long, or shorter where that leaves the
-// chip short of workgroups (z_chunks).
-constexpr int kRhsRowsMaxNx = 512;
+// row-marching RHS: one workgroup per (row segment, group of rows j, k chunk).
+// A workgroup of ty rows reads a neighbour row from HBM only for its first and
+// last row; a segment of tx threads has tx - 6 columns of its own.  The shapes by
+// row length (RHS alone, us, without / with the scalar):
+//   nx <= 64: whole rows, four per workgroup (64x48x64: 11.0 / 14.4 against 13.4
+//     / 17.1 with two; 64x128x64: 19 / 25 against 23 / 31);
+//   <= 128: whole rows, two (128x96x128: 42 / 55 against 47 / 63 with four);
+//   <= 244: two segments of 128 threads, two rows: four wavefronts, so two
+//     workgroups share a CU (240x64x96: 42 / 56 against 47 / 65 for whole rows;
+//     192x96x128: 66 / 85 against 63 / 100);
+//   <= 256: whole rows, two (256x128x192: 158 / 215 against 200 / 264, three
+//     segments would idle a third of the lanes);
+//   <= 512: segments of 128 threads, two rows (280x76x210: 137 / 187 against 197
+//     / 304 for whole rows, 512x128x256: 458 / 618 against 464 / 908), or whole
+//     rows, one per workgroup, where the grid is too small for 1.5 such
+//     workgroups per CU;
+//   longer: segments of 128 threads; two rows while a field fits the last-level
+//     cache (1024x128x160: 533 / 731 against 587 / 778 with four; 768x128x192:
+//     497 / 674 against 545 / 711), four beyond it, where the re-read edge rows
+//     come from HBM (4608x140x350: 5650 / 7470 against 6160 / 8050 with two), and
+//     four on the smallest grids.
+// The k chunks are many enough for about 96 wavefronts per CU over the launch
+// (more rounds of resident workgroups, so the partial last one costs less) and at
+// least 16 planes long, or shorter where that leaves the chip short of workgroups
+// (z_chunks).
 constexpr int kRhsSegThreads = 128;
 constexpr int kRhsXcdRun = 32;
 constexpr int kRhsMinPlanes = 16;
+constexpr size_t kRhsCachedField = size_t(256) << 20;
 struct RhsShape {
   int tx, ty, seg, run, minpl, nseg, nyb, nch;
 };
@@ -1066,17 +1082,22 @@ static int z_chunks(int nz, long long tiles, int want, int minpl, bool shrink, i
 }
 static RhsShape rhs_shape(const ptc_ctx *c) {
   RhsShape s{};
-  if (c->nx <= kRhsRowsMaxNx) {
+  const int cols = kRhsSegThreads - 6, nseg = (c->nx + cols - 1) / cols;
+  // 1.5 workgroups per CU with two-row segments and chunks of 16 planes
+  const bool enough = 2LL * nseg * ((c->ny + 1) / 2) * std::max(1, c->nz / kRhsMinPlanes) >= 3LL * c->n_cu;
+  const bool whole = c->nx <= 128 || (c->nx > 2 * cols && c->nx <= 256) || (c->nx > 256 && c->nx <= 512 && !enough);
+  if (whole) {
     s.tx = (c->nx + 63) / 64 * 64;
     s.seg = 0;
   } else {
     s.tx = c->rhs_seg_req ? c->rhs_seg_req : kRhsSegThreads;
     s.seg = s.tx - 6;
   }
-  // rows per workgroup: four for segmented rows (the RHS alone at
-  // 4608x140x700 15.7 against 16.1 ms with two, at 1536x192x256 2.71 against
-  // 2.74), two for whole rows of at most 128 points, else one
-  const int ty = c->rhs_rows_req ? c->rhs_rows_req : (s.seg ? 4 : (s.tx <= 128 ? 2 : 1));
+  int ty;
+  if (whole) ty = s.tx == 64 ? 4 : (c->nx <= 256 ? 2 : 1);
+  else if (c->nx <= 512) ty = 2;
+  else ty = enough && sizeof(double) * c->n3 <= kRhsCachedField ? 2 : 4;
+  if (c->rhs_rows_req) ty = c->rhs_rows_req;
   s.ty = std::max(1, std::min({ty, 512 / s.tx, c->ny}));
   s.run = c->rhs_run_req ? c->rhs_run_req : kRhsXcdRun;
   s.nseg = s.seg ? (c->nx + s.seg - 1) / s.seg : 1;
@@ -1148,16 +1169,19 @@ int launch_rhs(ptc_ctx *c, const double *ux, const double *uy, const double *uz,
   const RhsShape sh = rhs_shape(c);
   const int nt = sh.tx * sh.ty;
   const int lw = sh.seg ? sh.tx : c->nx;  // LDS row width
-  const size_t lds = sizeof(double) * (size_t)std::max(X_NROWS * sh.ty * lw, nt);
-#define PTC_ROWS(SCAL, MAXT)                                                                                  \
-  hipLaunchKernelGGL((k_rhs_rows<SCAL, MAXT>), grid, dim3(sh.tx, sh.ty), lds, c->stream, c->geo, cf, kc, ux, uy, \
+  const size_t lds = sizeof(double) * (size_t)std::max(X_NROWS * (sh.ty + 2) * lw, nt);
+#define PTC_ROWS(SCAL, MAXT, ONE)                                                                             \
+  hipLaunchKernelGGL((k_rhs_rows<SCAL, MAXT, ONE>), grid, dim3(sh.tx, sh.ty), lds, c->stream, c->geo, cf, kc, ux, uy, \
                      uz, sc, p, rhsx, rhsy, rhsz, rhsc, hx, hy, hz, hc, c->d_red, sh.seg, lw, sh.run)
-  if (nt <= 256) {
-    if (cf.scalar) PTC_ROWS(true, 256);
-    else PTC_ROWS(false, 256);
+  if (sh.ty == 1) {
+    if (cf.scalar) PTC_ROWS(true, 512, true);
+    else PTC_ROWS(false, 512, true);
+  } else if (nt <= 256) {
+    if (cf.scalar) PTC_ROWS(true, 256, false);
+    else PTC_ROWS(false, 256, false);
   } else {
-    if (cf.scalar) PTC_ROWS(true, 512);
-    else PTC_ROWS(false, 512);
+    if (cf.scalar) PTC_ROWS(true, 512, false);
+    else PTC_ROWS(false, 512, false);
   }
 #undef PTC_ROWS
   PTC_HIP(hipGetLastError());
