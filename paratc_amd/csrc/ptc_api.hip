@@ -300,6 +300,8 @@ int channel_step(ptc_ctx *c, double *mon) {
   double dt = c->prm.dtmax, uddxmax = 0.0;
   Monitors mo{};
   const bool adaptive = c->prm.icfl == 1;
+  PTC_TRY(poisson_build_plan(c));
+  PTC_TRY(stencil_prepare(c));  // no partials move between the monitors and their reading
   if (adaptive || mon) PTC_TRY(launch_monitors(c, kMonCfl, ux, uy, uz));
   if (adaptive) {
     PTC_TRY(read_monitors(c, kMonCfl, &mo));
@@ -325,7 +327,6 @@ int channel_step(ptc_ctx *c, double *mon) {
     // else written to RealArr1 first.  Its maximum is reduced only where it is
     // read (the last substep's, reported by the monitors).
     if (poisson_div_fusable(c)) {
-      PTC_TRY(stencil_prepare(c));  // partials for the x pass's workgroups (already sized under capture)
       const DivSrc dv{ux, uy, uz, 1.0 / c->pmAlpha, c->d_red};
       PTC_TRY(poisson_solve_div(c, dv, hl, true));
       if (ns == c->iadvance) PTC_TRY(launch_divmax(c, (int)fft_x_fwd_blocks(c, c->ny)));

@@ -163,7 +163,7 @@ struct ptc_ctx {
   double *d_red = nullptr;     // reduction partials
   int red_cap = 0;
   double *d_scal = nullptr;    // device scalars
-  double *d_mon = nullptr;     // partial maxima of the monitors
+  double *d_mon = nullptr;     // partial maxima of the monitors, behind the partials of d_red
   double *d_cnfac = nullptr;   // Crank-Nicolson factor tables (kCnMaxJobs + kCnStepTables) x kCnFacStride
   // beta each step table (substep ns, kind) holds, NaN when none; the tables
   // also depend on the chunk plan (cn_tab_mm, cn_tab_p) and the metrics

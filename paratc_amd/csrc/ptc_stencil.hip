@@ -1127,6 +1127,15 @@ static int rhs_nblocks(const ptc_ctx *c) {
   return (int)(gr.x * gr.y * gr.z);
 }
 
+static dim3 vel_grid(const ptc_ctx *c, int *kc);
+
+// workgroups of a monitor pass
+static int mon_nblocks(const ptc_ctx *c) {
+  int kc = 0;
+  const dim3 gr = vel_grid(c, &kc);
+  return (int)(gr.x * gr.y * gr.z);
+}
+
 int ensure_red(ptc_ctx *c, int n) {
   if (c->red_cap < n) {
     // a captured step (this context's or an ensemble's) holds the old address
@@ -1134,8 +1143,11 @@ int ensure_red(ptc_ctx *c, int n) {
     ++c->buf_gen;
     if (c->d_red) (void)hipFree(c->d_red);
     c->d_red = nullptr;
+    c->d_mon = nullptr;
     c->red_cap = 0;
-    PTC_HIP(hipMalloc(&c->d_red, sizeof(double) * (size_t)n));
+    // the monitors' partials follow: they outlive a step's launches
+    PTC_HIP(hipMalloc(&c->d_red, sizeof(double) * ((size_t)n + (size_t)kMonitors * mon_nblocks(c))));
+    c->d_mon = c->d_red + n;
     c->red_cap = n;
   }
   return PTC_OK;
@@ -1403,13 +1415,13 @@ int launch_uy_ym(ptc_ctx *c, double *uy_ym, double *duy_ym) {
 }
 
 // Enqueue the pass over the velocities that forms the asked maxima (kMon...);
-// read_monitors later brings them to the host.  The partials have their own
-// buffer, so a step may run in between.
+// read_monitors later brings them to the host.  The partials have their own part
+// of the reduction buffer, so a step whose partials are sized (stencil_prepare)
+// may run in between.
 int launch_monitors(ptc_ctx *c, int what, const double *ux, const double *uy, const double *uz) {
   int kc = 0;
   const dim3 grid = vel_grid(c, &kc);
-  const int nb = (int)(grid.x * grid.y * grid.z);
-  if (!c->d_mon) PTC_HIP(hipMalloc(&c->d_mon, sizeof(double) * (size_t)nb * kMonitors));
+  PTC_TRY(ensure_red(c, 1));
 #define PTC_MON(C, D, V)                                                                                      \
   hipLaunchKernelGGL((k_monitors<C, D, V>), grid, dim3(64, 4), 0, c->stream, c->geo, ux, uy, uz, kc, kVelXcdRun, \
                      c->d_mon)
@@ -1426,9 +1438,7 @@ int launch_monitors(ptc_ctx *c, int what, const double *ux, const double *uy, co
 // The maxima of `what` (any of the kMon... sets launched since the last read)
 // and clcPrSrc's divergence maximum on the host (synchronises)
 int read_monitors(ptc_ctx *c, int what, Monitors *out) {
-  int kc = 0;
-  const dim3 grid = vel_grid(c, &kc);
-  const int nb = (int)(grid.x * grid.y * grid.z);
+  const int nb = mon_nblocks(c);
   const int q0 = what & kMonCfl ? 0 : (what & kMonDiv ? 1 : 2);
   const int q1 = what & kMonVmax ? 5 : (what & kMonDiv ? 2 : 1);
   double *h = c->h_pinned + kPinMonitors;
@@ -1545,7 +1555,7 @@ __global__ void __launch_bounds__(256, 2) k_stat_rows(Geo g, double ucrf, const 
   const bool wall = by + 1 == nyb;
   const int jrow = wall ? ny + 1 : by * nr + r + 1;
   const bool live = wall ? r == 0 : jrow <= ny;
-  const int j = wall ? ny + 1 : min(jrow, ny), jm = j - 1, jp = j + 1;
+  const int j = wall ? ny + 1 : min(jrow, ny), jp = j + 1;
   const double IY1 = met[M_YINT * nyh + j], IY2 = 1.0 - IY1;
   const double cac = met[M_RDYC * nyh + j];
   auto wz = [&](int kk) { return (long long)(kk < 0 ? kk + nz : (kk >= nz ? kk - nz : kk)) * g.plane; };

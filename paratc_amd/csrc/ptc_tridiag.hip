@@ -609,22 +609,19 @@ __global__ void __launch_bounds__(64) k_cn_factor(CnJobs jobs, const double *__r
 
 // The constant-flow-rate shift of RhsX (src/m_TScheme.f90:269-300), in the
 // arithmetic of k_flowrate: every workgroup of the u job sums the RHS
-// kernel's partials in the same fixed order (strided per thread, then a tree
-// in red), so all hold the same shift; workgroup (0, 0) stores it and the
+// kernel's partials in the same fixed order (strided per thread, across the
+// wavefront, then the wavefronts in red), so all hold the same shift; workgroup (0, 0) stores it and the
 // PrGradAver increment, as k_flowrate would.  Called by all threads.
 __device__ double flow_fold_shift(const FlowFold &ff, double *red) {
   const int t = threadIdx.x, nt = blockDim.x;
   double acc = 0.0;
   for (int q = t; q < ff.n; q += nt) acc += ff.part[q];
-  red[t] = acc;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+  if ((t & 63) == 0) red[t >> 6] = acc;
   __syncthreads();
-  for (int n = nt; n > 1;) {
-    const int h = (n + 1) / 2;
-    if (t < n - h) red[t] += red[t + h];
-    __syncthreads();
-    n = h;
-  }
-  const double tot = red[0];
+  double tot = 0.0;
+  for (int w = 0; w < (nt + 63) / 64; ++w) tot += red[w];
   __syncthreads();  // red is the solve's LDS
   double shift, inc;
   if (ff.scalar_build) {
@@ -759,7 +756,12 @@ struct TriShape {
 };
 static const TriShape kPoissonShapes[] = {{4, 64, 1024}, {8, 64, 1024}, {12, 64, 1024}, {16, 64, 1024},
                                           {8, 32, 1024},  {12, 32, 1024}, {16, 32, 512},  {16, 16, 256}};
-static const TriShape kCnShapes[] = {{4, 64, 1024}, {8, 64, 1024}, {12, 64, 1024}, {8, 32, 1024}, {16, 32, 512}};
+// Crank-Nicolson chunks of 12 rows first: fewer cyclic-reduction steps and, at
+// 512 threads for ny = 96, three workgroups per CU where 8-row chunks' 768 threads
+// leave a round of workgroups half empty (RK substep 128x96x128 144.8 -> 139.3 us,
+// 256x128x192 486 -> 472, 280x76x210 423 -> 413); above 192 rows chunks of 16
+// (64x256x64 114 -> 112).
+static const TriShape kCnShapes[] = {{12, 64, 1024}, {8, 64, 1024}, {4, 64, 1024}, {16, 32, 512}, {8, 32, 1024}};
 
 static int tri_choose(int ny, size_t lds_limit, int mm_req, int lpb_req, const TriShape *shapes, int nshapes,
                       int *P_out, int *mm_out, int *lpb_out) {
