@@ -140,8 +140,9 @@ struct SpectraState {
   double *d_x = nullptr, *d_z = nullptr, *d_2d = nullptr;
   int pitch = 0, nch = 0;                      // spectral row pitch and kz chunks of the work buffers
   double2 *d_fa = nullptr, *d_fb = nullptr;    // FP64 2-D spectra pitch * ny * nz
-  double *d_cell = nullptr;                    // cell-centre field, field layout
-  double2 *d_px = nullptr, *d_pz = nullptr;    // partial sums
+  double *d_toprow = nullptr;                  // uy's row ny+1 as a field of one row
+  double2 *d_top = nullptr;                    // its 2-D spectrum, pitch * nz
+  double *d_px = nullptr, *d_pz = nullptr;     // partial sums
   double2 *d_hx = nullptr;                     // symbol of the cell-centre interpolation of ux
 };
 
@@ -426,6 +427,32 @@ int launch_monitors(ptc_ctx *c, int what, const double *ux, const double *uy, co
 int read_monitors(ptc_ctx *c, int what, Monitors *out);
 int launch_monitor_sum(ptc_ctx *c, int which, const double *ux, const double *s, double *out);
 int reduce_sum_s3(ptc_ctx *c, int nparts, double *host_out);
+
+// Sums NS values over a wavefront: each of six exchanges sends half of the values
+// a lane still holds to the lane that keeps them, so NS values cost about NS
+// exchanges instead of 6 NS.  On return lane l holds the sum of value *idx in
+// v[0] (*idx = -1: none).  Fixed order.
+template <int NS, int N, int MASK>
+__device__ __forceinline__ void wave_sums_step(double (&v)[NS], int lane, int &base, int &count) {
+  constexpr int H = (N + 1) / 2;
+  const bool up = lane & MASK;
+#pragma unroll
+  for (int q = 0; q < H; ++q) {
+    const double hi = q + H < N ? v[q + H] : 0.0;
+    const double send = up ? v[q] : hi, keep = up ? hi : v[q];
+    v[q] = keep + __shfl_xor(send, MASK);
+  }
+  base += up ? H : 0;
+  count = up ? count - H : min(count, H);
+  if constexpr (MASK > 1) wave_sums_step<NS, H, MASK / 2>(v, lane, base, count);
+}
+template <int NS>
+__device__ __forceinline__ void wave_sums(double (&v)[NS], int lane, int *idx) {
+  static_assert(NS <= 64, "one value per lane at the end");
+  int base = 0, count = NS;
+  wave_sums_step<NS, NS, 32>(v, lane, base, count);
+  *idx = count > 0 ? base : -1;
+}
 
 // The partial results of a launch reduced by one workgroup of
 // kReduceThreads threads: every thread has eight loads in flight (indices past

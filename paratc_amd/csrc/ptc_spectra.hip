@@ -23,7 +23,8 @@
 // (the 4-point interpolation ic1 ux(i-1) + ic2 ux(i) + ic3 ux(i+1) + ic4 ux(i+2)
 // + uCRF) is not transformed separately: its spectrum is H(kx) F_ux(kx, kz)
 // with H = ic1 w + ic2 + ic3 conj(w) + ic4 conj(w)^2, w = exp(-2 pi i kx / nx),
-// plus the same shift.
+// plus the same shift.  Nor is the cell-centre uy, the mean of two face rows: its
+// spectrum is the mean of theirs (uy's row ny+1 is transformed by itself).
 #include "ptc_internal.hpp"
 
 #include <algorithm>
@@ -33,173 +34,178 @@ namespace ptc {
 
 namespace {
 
-constexpr int kSpecThreads = 256;  // partial-sum workgroup
+constexpr int kSpecThreads = 320;  // largest partial-sum workgroup: 257 kx (nx = 512) fit one per thread
 constexpr int kSpecRows = 16;      // kz rows per partial-sum workgroup
 
-// ---- the cell-centre uy (:576-587): the two-face mean into rows 1..ny of a field
-__global__ void __launch_bounds__(256) k_spec_cell(Geo g, const double *__restrict__ u, double *__restrict__ out) {
-  const int i = blockIdx.x * 256 + threadIdx.x, j = 1 + blockIdx.y, k = blockIdx.z;
-  if (i >= g.nx) return;
-  const long long o = (long long)g.nx * j + g.plane * k + i;
-  out[o] = 0.5 * (u[o] + u[o + g.nx]);
+// ---- row ny+1 of a field as row 1 of a field of one row
+__global__ void __launch_bounds__(256) k_spec_top(Geo g, const double *__restrict__ u, double *__restrict__ out) {
+  const int i = blockIdx.x * 256 + threadIdx.x, k = blockIdx.y;
+  if (i < g.nx) out[(long long)g.nx * (3LL * k + 1) + i] = u[(long long)g.nx * (g.ny + 1) + g.plane * k + i];
 }
 
 __device__ inline double2 cmul(double2 a, double2 b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
 
-// One pair of spectra to multiply, P = Fa conj Fb.  b's row is the same row,
-// or (lcs) the reference row: jr1 below row jsplit, jr2 from it on.  ha: a is
-// first multiplied by hx[kx] (the cell-centre interpolation's symbol).
-struct SpecPair {
-  const double2 *a, *b;
-  double sa, sb;  // added to Re F(0, 0) of a and b (after the multiplication)
-  int lcs, jr1, jr2, jsplit;
-  const double2 *ha;
+// The products of one field's spectrum a, summed over kz and over kx.  kEnergy:
+// |a|^2.  kSet (a = ux): |a|^2; a conj a(reference row jr1 below row jsplit, jr2
+// from it on), complex; a conj c and (hx a) conj c, real parts, with c the
+// cell-centre uy from the rows j and j+1 of v (vtop for row ny+1).  sa is added to
+// Re F(0, 0) of a (after the multiplication by hx).
+enum { kEnergy = 0, kSet = 1 };
+struct SpecIn {
+  const double2 *a, *v, *vtop, *hx;
+  double sa;
+  int jr1, jr2, jsplit;
 };
+// products formed as sums over kz per kx (px), and sums over all kx and over
+// 0 < kx < h per kz (pz: two per product)
+constexpr int spec_products(int mode) { return mode == kEnergy ? 1 : 5; }
 
-// Partial sums of one row j and kSpecRows kz rows (grid: x = kz chunk, y = j):
-//   px[(j * nch + chunk) * (h+1) + kx] = sum over the chunk's kz of P(kx, kz)
-//   pz[2 * (j * nz + kz)]     = sum over kx = 0..h of P(kx, kz)
-//   pz[2 * (j * nz + kz) + 1] = sum over kx = 1..h-1 of P(kx, kz)
-// Thread t owns kx = t + 256 s, s < NS.  Rows go in batches of spec_batch
-// (fewer for more kx per thread, to stay within the registers): all their
-// loads are issued before the products and the wavefront sums.
-template <int NS>
-constexpr int spec_batch() { return NS == 1 ? 4 : NS <= 3 ? 2 : 1; }
+// Partial sums of one row j, kSpecRows kz rows and a segment of kx (grid: x = kz
+// chunk, y = j, z = segment of blockDim * NS kx):
+//   px[((q * ny + j) * nch + chunk) * (h+1) + kx]       = sum over the chunk's kz
+//   pz[(((2 q + inner) * ny + j) * nz + kz) * nseg + seg] = sum over the segment's
+//                                            kx, all or only those in 1..h-1
+// of product q.  Thread t owns kx = seg start + t + blockDim s, s < NS.  All
+// products of a field come from one read of its spectrum, and the sums over kx of
+// a batch of rows are exchanged together (wave_sums): one product per launch with
+// six exchanges per value read the ux and uy spectra seven times and took 78 us
+// a product at 512x128x256, where one read takes about 27.
+constexpr int kSpecMaxNs = 4;
+template <int NS, int MODE>
+constexpr int spec_batch() {
+  return MODE == kEnergy ? (NS == 1 ? 8 : NS <= 2 ? 4 : 2) : (NS == 1 ? 4 : NS <= 2 ? 2 : 1);
+}
 
-template <int NS, bool SAME>
-__global__ void __launch_bounds__(kSpecThreads) k_spec_part(SpecPair P, int ny, int nz, int h, int pitch,
-                                                            double2 *__restrict__ px, double2 *__restrict__ pz) {
-  constexpr int NW = kSpecThreads / 64, RB = spec_batch<NS>();
-  __shared__ double red[kSpecRows][NW][4];
+template <int NS, int MODE>
+__global__ void __launch_bounds__(kSpecThreads) k_spec_sums(SpecIn S, int ny, int nz, int h, int pitch,
+                                                            double *__restrict__ px, double *__restrict__ pz) {
+  constexpr int NW = kSpecThreads / 64, NQ = spec_products(MODE), RB = spec_batch<NS, MODE>(), NV = 2 * NQ;
+  __shared__ double red[kSpecRows][NW][NV];
   const int j = blockIdx.y, ch = blockIdx.x, nch = gridDim.x;
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int t = threadIdx.x, nt = blockDim.x, lane = t & 63, w = t >> 6, nw = nt >> 6;
   const int k0 = ch * kSpecRows, k1 = min(nz, k0 + kSpecRows);
-  const int jb = P.lcs ? (j < P.jsplit ? P.jr1 : P.jr2) : j;
-  double sxr[NS], sxi[NS];
+  const int kx0 = (int)blockIdx.z * nt * NS + t;
+  const int jr = j < S.jsplit ? S.jr1 : S.jr2;
+  double sx[NS][NQ];
   double2 hs[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const int kx = t + kSpecThreads * s;
-    sxr[s] = sxi[s] = 0.0;
-    hs[s] = (P.ha && kx <= h) ? P.ha[kx] : make_double2(1.0, 0.0);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) sx[s][q] = 0.0;
+    if (MODE == kSet) hs[s] = S.hx[min(kx0 + nt * s, h)];
   }
+  struct Row {
+    double2 a, b, v0, v1;
+  };
+  auto load = [&](int kz, int kx) {
+    Row r{};
+    const long long base = (long long)kz * ny;
+    r.a = S.a[(base + j) * pitch + kx];
+    if constexpr (MODE == kSet) {
+      r.b = S.a[(base + jr) * pitch + kx];
+      r.v0 = S.v[(base + j) * pitch + kx];
+      r.v1 = j + 1 < ny ? S.v[(base + j + 1) * pitch + kx] : S.vtop[(long long)kz * pitch + kx];
+    }
+    return r;
+  };
+  // the products of one mode into the sums over kz and the row's values
+  auto add = [&](const Row &r, int kz, int kx, double2 hx, double (&s)[NQ], double *v) {
+    double2 a = r.a;
+    const bool origin = kz == 0 && kx == 0;
+    double pr[NQ];
+    if constexpr (MODE == kSet) {
+      double2 b = r.b, ha = cmul(a, hx);
+      if (origin) {
+        b.x += S.sa;
+        ha.x += S.sa;
+      }
+      const double2 c = make_double2(0.5 * (r.v0.x + r.v1.x), 0.5 * (r.v0.y + r.v1.y));
+      if (origin) a.x += S.sa;
+      pr[1] = a.x * b.x + a.y * b.y;
+      pr[2] = a.y * b.x - a.x * b.y;
+      pr[3] = a.x * c.x + a.y * c.y;
+      pr[4] = ha.x * c.x + ha.y * c.y;
+    }
+    pr[0] = a.x * a.x + a.y * a.y;
+    const bool inner = kx > 0 && kx < h;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      s[q] += pr[q];
+      v[2 * q] += pr[q];
+      v[2 * q + 1] += inner ? pr[q] : 0.0;
+    }
+  };
   for (int kb = k0; kb < k1; kb += RB) {
-    double2 va[RB][NS], vb[RB][NS];
+    Row row[RB][NS];
 #pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      const bool live = kb + r < k1;
-      const long long kz = live ? kb + r : k0;
-      const double2 *ra = P.a + (kz * ny + j) * pitch;
-      const double2 *rb = P.b + (kz * ny + jb) * pitch;
+    for (int r = 0; r < RB; ++r)
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const int kx = t + kSpecThreads * s;
-        const bool in = live && kx <= h;
-        va[r][s] = in ? ra[kx] : make_double2(0.0, 0.0);
-        if (!SAME) vb[r][s] = in ? rb[kx] : make_double2(0.0, 0.0);
-      }
-    }
-    double q[RB][4];
+      for (int s = 0; s < NS; ++s) row[r][s] = load(min(kb + r, k1 - 1), min(kx0 + nt * s, h));
+    double q[RB * NV];
 #pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      q[r][0] = q[r][1] = q[r][2] = q[r][3] = 0.0;
-      const bool origin = kb + r == 0;
+    for (int e = 0; e < RB * NV; ++e) q[e] = 0.0;
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const int kx = t + kSpecThreads * s;
-        double2 a = P.ha ? cmul(va[r][s], hs[s]) : va[r][s];
-        if (origin && kx == 0) a.x += P.sa;
-        double2 b = a;
-        if (!SAME) {
-          b = vb[r][s];
-          if (origin && kx == 0) b.x += P.sb;
-        }
-        const double pr = a.x * b.x + a.y * b.y, pi = a.y * b.x - a.x * b.y;
-        sxr[s] += pr;
-        sxi[s] += pi;
-        q[r][0] += pr;
-        q[r][1] += pi;
-        if (kx > 0 && kx < h) {
-          q[r][2] += pr;
-          q[r][3] += pi;
-        }
-      }
-    }
+    for (int r = 0; r < RB; ++r)
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-      for (int r = 0; r < RB; ++r)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) q[r][e] += __shfl_xor(q[r][e], off);
-    if (lane == 0) {
-#pragma unroll
-      for (int r = 0; r < RB; ++r)
-        if (kb + r < k1)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) red[kb + r - k0][w][e] = q[r][e];
-    }
+      for (int s = 0; s < NS; ++s)
+        if (kb + r < k1 && kx0 + nt * s <= h) add(row[r][s], kb + r, kx0 + nt * s, hs[s], sx[s], q + r * NV);
+    int idx;
+    wave_sums<RB * NV>(q, lane, &idx);
+    if (idx >= 0 && kb + idx / NV < k1) red[kb - k0 + idx / NV][w][idx % NV] = q[0];
   }
-  double2 *ox = px + ((long long)j * nch + ch) * (h + 1);
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int kx = t + kSpecThreads * s;
-    if (kx <= h) ox[kx] = make_double2(sxr[s], sxi[s]);
+  for (int q = 0; q < NQ; ++q) {
+    double *ox = px + (((long long)q * ny + j) * nch + ch) * (h + 1);
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      if (kx0 + nt * s <= h) ox[kx0 + nt * s] = sx[s][q];
   }
   __syncthreads();
-  if (t < k1 - k0) {
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int qq = 0; qq < NW; ++qq)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] += red[t][qq][e];
-    double2 *oz = pz + 2 * ((long long)j * nz + k0 + t);
-    oz[0] = make_double2(v[0], v[1]);
-    oz[1] = make_double2(v[2], v[3]);
+  for (int e = t; e < (k1 - k0) * NV; e += nt) {
+    const int r = e / NV, v = e - r * NV;
+    double sum = 0.0;
+    for (int qw = 0; qw < nw; ++qw) sum += red[r][qw][v];
+    pz[(((long long)v * ny + j) * nz + k0 + r) * gridDim.z + blockIdx.z] = sum;
   }
 }
 
-// Adds one sample to the 1-D accumulators of row j (grid: y = j).
-//   kind 0: energy or co-spectrum (weight 2 inside, 1 at kx = 0, nx/2),
-//           real part into quantity m0;
-//   kind 1: linear coherence, real part into m0 and imaginary part (zero at
-//           the edge wavenumbers) into m1, no weight.
-// ex(kx, j, m) and ez(kz, j, m) are column-major as EnergySpecX/Z.
-__global__ void __launch_bounds__(256) k_spec_fin(const double2 *__restrict__ px, const double2 *__restrict__ pz,
-                                                  int nch, int ny, int nx, int nz, int kind, int m0, int m1,
+// Adds one sample to the 1-D accumulators (grid: x = product, y = row j).
+// Products of kEnergy: an energy into quantity m (weight 2 inside, 1 at kx = 0,
+// nx/2).  Products of kSet: the energy (1), the linear coherence's real (7) and
+// imaginary part (8, zero at the edge wavenumbers), no weight, and two
+// co-spectra (5, 6), weighted.  ex(kx, j, m) and ez(kz, j, m) are column-major as
+// EnergySpecX/Z; m is 1-based.
+__global__ void __launch_bounds__(256) k_spec_fin(const double *__restrict__ px, const double *__restrict__ pz,
+                                                  int nch, int nseg, int ny, int nx, int nz, int mode, int m,
                                                   double *__restrict__ ex, double *__restrict__ ez) {
-  const int j = blockIdx.y, h = nx / 2, nzh = nz / 2;
+  const int j = blockIdx.y, q = blockIdx.x, h = nx / 2, nzh = nz / 2;
+  const bool imag = mode == kSet && q == 2, coh = mode == kSet && (q == 1 || q == 2);
+  constexpr int set_m[5] = {1, 7, 8, 5, 6};
+  const int m0 = (mode == kSet ? set_m[q] : m) - 1;
   // normEgy of the x and z helpers (:962, :1048)
   const double normx = 1.0 / ((double)nx * (double)nx * (double)nz);
   const double normz = 1.0 / ((double)nx * (double)nz * (double)nz);
+  const double *pq = px + ((long long)q * ny + j) * nch * (h + 1);
   for (int kx = threadIdx.x; kx <= h; kx += blockDim.x) {
-    double sr = 0.0, si = 0.0;
-    for (int c = 0; c < nch; ++c) {
-      const double2 v = px[((long long)j * nch + c) * (h + 1) + kx];
-      sr += v.x;
-      si += v.y;
-    }
+    const bool edge = kx == 0 || kx == h;
+    if (imag && edge) continue;
+    double sr = 0.0;
+    for (int c = 0; c < nch; ++c) sr += pq[(long long)c * (h + 1) + kx];
     sr = sr / (double)nz;
-    si = si / (double)nz;
-    double *o0 = ex + kx + (long long)(h + 1) * (j + (long long)ny * m0);
-    if (kind == 0) {
-      *o0 += sr * ((kx == 0 || kx == h) ? 1.0 : 2.0) * normx;
-    } else {
-      *o0 += sr * normx;
-      if (kx > 0 && kx < h) ex[kx + (long long)(h + 1) * (j + (long long)ny * m1)] += si * normx;
-    }
+    ex[kx + (long long)(h + 1) * (j + (long long)ny * m0)] += sr * (coh || edge ? 1.0 : 2.0) * normx;
   }
+  auto zsum = [&](int in, int kz) {
+    const double *pq2 = pz + (((long long)(2 * q + in) * ny + j) * nz + kz) * nseg;
+    double s = 0.0;
+    for (int g = 0; g < nseg; ++g) s += pq2[g];
+    return s;
+  };
   for (int kz = threadIdx.x; kz <= nzh; kz += blockDim.x) {
-    const double2 r = pz[2 * ((long long)j * nz + kz)];
+    const bool edge = kz == 0 || kz == nzh;
+    if (imag && edge) continue;
     const int km = kz == 0 ? 0 : nz - kz;
-    const double2 q = pz[2 * ((long long)j * nz + km) + 1];
-    const double vr = (r.x + q.x) / (double)nx, vi = (r.y - q.y) / (double)nx;
-    double *o0 = ez + kz + (long long)(nzh + 1) * (j + (long long)ny * m0);
-    if (kind == 0) {
-      *o0 += vr * ((kz == 0 || kz == nzh) ? 1.0 : 2.0) * normz;
-    } else {
-      *o0 += vr * normz;
-      if (kz > 0 && kz < nzh) ez[kz + (long long)(nzh + 1) * (j + (long long)ny * m1)] += vi * normz;
-    }
+    const double v = (imag ? zsum(0, kz) - zsum(1, km) : zsum(0, kz) + zsum(1, km)) / (double)nx;
+    ez[kz + (long long)(nzh + 1) * (j + (long long)ny * m0)] += v * (coh || edge ? 1.0 : 2.0) * normz;
   }
 }
 
@@ -207,16 +213,21 @@ __global__ void __launch_bounds__(256) k_spec_fin(const double2 *__restrict__ px
 // spectral row `row` (0-based): p <= h is the real part of the x transform at
 // kx = p, p > h its imaginary part at kx = nx - p; q likewise along z.
 // hx (may be null) multiplies F first and shift is then added to Re F(0, 0).
-__device__ inline double hc2d_value(const double2 *__restrict__ F, const double2 *__restrict__ hx, double shift,
-                                    int ny, int nx, int nz, int pitch, int row, int p, int q) {
+// cell: the mean of rows row and row+1 (top past row ny-1).
+__device__ inline double hc2d_value(const double2 *__restrict__ F, const double2 *__restrict__ top, bool cell,
+                                    const double2 *__restrict__ hx, double shift, int ny, int nx, int nz, int pitch,
+                                    int row, int p, int q) {
   const int h = nx / 2, nzh = nz / 2;
   const int kx = p <= h ? p : nx - p, kz = q <= nzh ? q : nz - q, km = kz == 0 ? 0 : nz - kz;
-  double2 f1 = F[((long long)kz * ny + row) * pitch + kx];
-  double2 f2 = F[((long long)km * ny + row) * pitch + kx];
-  if (hx) {
-    f1 = cmul(f1, hx[kx]);
-    f2 = cmul(f2, hx[kx]);
-  }
+  auto at = [&](int k) {
+    double2 f = F[((long long)k * ny + row) * pitch + kx];
+    if (cell) {
+      const double2 g = row + 1 < ny ? F[((long long)k * ny + row + 1) * pitch + kx] : top[(long long)k * pitch + kx];
+      f = make_double2(0.5 * (f.x + g.x), 0.5 * (f.y + g.y));
+    }
+    return hx ? cmul(f, hx[kx]) : f;
+  };
+  double2 f1 = at(kz), f2 = at(km);
   if (kx == 0 && kz == 0) {
     f1.x += shift;
     f2.x += shift;
@@ -226,73 +237,68 @@ __device__ inline double hc2d_value(const double2 *__restrict__ F, const double2
 }
 
 // Adds one sample to the 2-D accumulator of quantity m (grid: x = p / 64,
-// y = chosen row, z = q).  mirror: 0 none (half channel), 1 the row ny+1-jct,
-// 2 the face row ny+2-jct (uy); rcoe weighs the mirror's product.
+// y = chosen row, z = q).  b is a's row, or (top not null) the cell-centre uy's.
+// mirror: 0 none (half channel), 1 the row ny+1-jct, 2 the face row ny+2-jct (uy);
+// rcoe weighs the mirror's product.
 __global__ void __launch_bounds__(64) k_spec_2d(const double2 *__restrict__ a, const double2 *__restrict__ b,
-                                                const double2 *__restrict__ ha, double sa, int ny, int nx, int nz,
-                                                int pitch, const int *__restrict__ iy, int ny2d, int mirror,
-                                                double rcoe, double norm, double *__restrict__ out) {
+                                                const double2 *__restrict__ top, const double2 *__restrict__ ha,
+                                                double sa, int ny, int nx, int nz, int pitch,
+                                                const int *__restrict__ iy, int ny2d, int mirror, double rcoe,
+                                                double norm, double *__restrict__ out) {
   const int p = blockIdx.x * 64 + threadIdx.x, jc = blockIdx.y, q = blockIdx.z;
   if (p >= nx) return;
   const int jct = iy[jc];
-  double v = hc2d_value(a, ha, sa, ny, nx, nz, pitch, jct - 1, p, q) *
-             hc2d_value(b, nullptr, 0.0, ny, nx, nz, pitch, jct - 1, p, q);
+  const bool cell = top != nullptr;
+  double v = hc2d_value(a, nullptr, false, ha, sa, ny, nx, nz, pitch, jct - 1, p, q) *
+             hc2d_value(b, top, cell, nullptr, 0.0, ny, nx, nz, pitch, jct - 1, p, q);
   if (mirror) {
     const int jcs = (mirror == 2 ? ny + 2 : ny + 1) - jct;
-    v += rcoe * (hc2d_value(a, ha, sa, ny, nx, nz, pitch, jcs - 1, p, q) *
-                 hc2d_value(b, nullptr, 0.0, ny, nx, nz, pitch, jcs - 1, p, q));
+    v += rcoe * (hc2d_value(a, nullptr, false, ha, sa, ny, nx, nz, pitch, jcs - 1, p, q) *
+                 hc2d_value(b, top, cell, nullptr, 0.0, ny, nx, nz, pitch, jcs - 1, p, q));
   }
   out[p + (long long)nx * (jc + (long long)ny2d * q)] += norm * v;
 }
 
+// launch shape of the partial sums: kx per thread, threads, segments of kx
+void sums_shape(int h, int *ns, int *nt, int *nseg) {
+  *ns = std::min(kSpecMaxNs, (h + kSpecThreads) / kSpecThreads);
+  *nt = std::min(kSpecThreads, ((h + *ns) / *ns + 63) / 64 * 64);
+  *nseg = (h + *nt * *ns) / (*nt * *ns);
+}
+
 template <int NS>
-void part_launch(ptc_ctx *c, const SpecPair &P, bool same, int nch, double2 *px, double2 *pz) {
-  const dim3 grid((unsigned)nch, (unsigned)c->ny);
-  if (same)
-    hipLaunchKernelGGL((k_spec_part<NS, true>), grid, dim3(kSpecThreads), 0, c->stream, P, c->ny, c->nz, c->nx / 2,
-                       c->spec.pitch, px, pz);
+void sums_launch(ptc_ctx *c, const SpecIn &S, int mode, int nt, int nseg) {
+  SpectraState &st = c->spec;
+  const dim3 grid((unsigned)st.nch, (unsigned)c->ny, (unsigned)nseg), blk((unsigned)nt);
+  if (mode == kSet)
+    hipLaunchKernelGGL((k_spec_sums<NS, kSet>), grid, blk, 0, c->stream, S, c->ny, c->nz, c->nx / 2, st.pitch, st.d_px,
+                       st.d_pz);
   else
-    hipLaunchKernelGGL((k_spec_part<NS, false>), grid, dim3(kSpecThreads), 0, c->stream, P, c->ny, c->nz, c->nx / 2,
-                       c->spec.pitch, px, pz);
+    hipLaunchKernelGGL((k_spec_sums<NS, kEnergy>), grid, blk, 0, c->stream, S, c->ny, c->nz, c->nx / 2, st.pitch,
+                       st.d_px, st.d_pz);
 }
 
-// kx values per thread, rounded up to an instantiated count
-int part_slots(int h) {
-  const int ns = (h + kSpecThreads) / kSpecThreads;
-  for (int n : {1, 2, 3, 4, 6, 10, 19})
-    if (ns <= n) return n;
-  return 0;
-}
-
-int launch_part(ptc_ctx *c, const SpecPair &P, bool same) {
+// the 1-D quantities of one field: kEnergy into quantity m (1-based as the
+// reference's), kSet into 1, 5, 6, 7, 8
+int spec_1d(ptc_ctx *c, const SpecIn &in, int mode, int m) {
   SpectraState &S = c->spec;
-  switch (part_slots(c->nx / 2)) {
-    case 1: part_launch<1>(c, P, same, S.nch, S.d_px, S.d_pz); break;
-    case 2: part_launch<2>(c, P, same, S.nch, S.d_px, S.d_pz); break;
-    case 3: part_launch<3>(c, P, same, S.nch, S.d_px, S.d_pz); break;
-    case 4: part_launch<4>(c, P, same, S.nch, S.d_px, S.d_pz); break;
-    case 6: part_launch<6>(c, P, same, S.nch, S.d_px, S.d_pz); break;
-    case 10: part_launch<10>(c, P, same, S.nch, S.d_px, S.d_pz); break;
-    case 19: part_launch<19>(c, P, same, S.nch, S.d_px, S.d_pz); break;
-    default: set_error("spectra: nx/2 above 4608"); return PTC_E_UNSUPPORTED;
+  int ns, nt, nseg;
+  sums_shape(c->nx / 2, &ns, &nt, &nseg);
+  switch (ns) {
+    case 1: sums_launch<1>(c, in, mode, nt, nseg); break;
+    case 2: sums_launch<2>(c, in, mode, nt, nseg); break;
+    case 3: sums_launch<3>(c, in, mode, nt, nseg); break;
+    default: sums_launch<4>(c, in, mode, nt, nseg); break;
   }
   PTC_HIP(hipGetLastError());
-  return PTC_OK;
-}
-
-// one 1-D quantity (kind 0, m0) or the linear-coherence pair (kind 1, m0, m1);
-// m are 1-based as the reference's
-int spec_1d(ptc_ctx *c, const SpecPair &P, bool same, int kind, int m0, int m1) {
-  SpectraState &S = c->spec;
-  PTC_TRY(launch_part(c, P, same));
-  hipLaunchKernelGGL(k_spec_fin, dim3(1, (unsigned)c->ny), dim3(256), 0, c->stream, S.d_px, S.d_pz, S.nch, c->ny,
-                     c->nx, c->nz, kind, m0 - 1, m1 - 1, S.d_x, S.d_z);
+  hipLaunchKernelGGL(k_spec_fin, dim3((unsigned)spec_products(mode), (unsigned)c->ny), dim3(256), 0, c->stream, S.d_px,
+                     S.d_pz, S.nch, nseg, c->ny, c->nx, c->nz, mode, m, S.d_x, S.d_z);
   PTC_HIP(hipGetLastError());
   return PTC_OK;
 }
 
 int spec_2d(ptc_ctx *c, const double2 *a, const double2 *b, int m, int mirror, double rcoe,
-            const double2 *ha = nullptr, double sa = 0.0) {
+            const double2 *top = nullptr, const double2 *ha = nullptr, double sa = 0.0) {
   SpectraState &S = c->spec;
   const int nx = c->nx, nz = c->nz;
   // normEgy of clcEnergySpectra2D / clcCosSpectra2D (:1253-1255)
@@ -301,15 +307,8 @@ int spec_2d(ptc_ctx *c, const double2 *a, const double2 *b, int m, int mirror, d
   if (c->prm.flow_type == 1) norm = norm * 0.5;
   double *out = S.d_2d + (long long)nx * S.ny2d * nz * (m - 1);
   const dim3 grid((unsigned)((nx + 63) / 64), (unsigned)S.ny2d, (unsigned)nz);
-  hipLaunchKernelGGL(k_spec_2d, grid, dim3(64), 0, c->stream, a, b, ha, sa, c->ny, nx, nz, S.pitch, S.d_iy2d, S.ny2d,
-                     c->prm.flow_type == 1 ? mirror : 0, rcoe, norm, out);
-  PTC_HIP(hipGetLastError());
-  return PTC_OK;
-}
-
-int cell_uy(ptc_ctx *c, const double *uy) {
-  const dim3 grid((unsigned)((c->nx + 255) / 256), (unsigned)c->ny, (unsigned)c->nz);
-  hipLaunchKernelGGL(k_spec_cell, grid, dim3(256), 0, c->stream, c->geo, uy, c->spec.d_cell);
+  hipLaunchKernelGGL(k_spec_2d, grid, dim3(64), 0, c->stream, a, b, top, ha, sa, c->ny, nx, nz, S.pitch, S.d_iy2d,
+                     S.ny2d, c->prm.flow_type == 1 ? mirror : 0, rcoe, norm, out);
   PTC_HIP(hipGetLastError());
   return PTC_OK;
 }
@@ -318,6 +317,17 @@ int cell_uy(ptc_ctx *c, const double *uy) {
 int forward(ptc_ctx *c, const double *src, double2 *spec) {
   PTC_TRY(launch_fft_x_fwd(c, src, spec, true));
   return launch_fft_z(c, spec, false, true);
+}
+
+// the 2-D spectrum of uy's row ny+1, through a context of one row
+int forward_top(ptc_ctx *c, const double *uy) {
+  SpectraState &S = c->spec;
+  hipLaunchKernelGGL(k_spec_top, dim3((unsigned)((c->nx + 255) / 256), (unsigned)c->nz), dim3(256), 0, c->stream, c->geo,
+                     uy, S.d_toprow);
+  PTC_HIP(hipGetLastError());
+  ptc_ctx one(*c);  // the launchers read its sizes and plan only
+  one.ny = 1;
+  return forward(&one, S.d_toprow, S.d_top);
 }
 
 template <typename T>
@@ -342,7 +352,8 @@ int ensure_work(ptc_ctx *c) {
   if (S.d_fa && S.pitch == c->pp.pitch) return PTC_OK;
   release(S.d_fa);
   release(S.d_fb);
-  release(S.d_cell);
+  release(S.d_toprow);
+  release(S.d_top);
   release(S.d_px);
   release(S.d_pz);
   release(S.d_hx);
@@ -351,9 +362,12 @@ int ensure_work(ptc_ctx *c) {
   const size_t nspec = (size_t)S.pitch * c->ny * c->nz;
   PTC_TRY(alloc(&S.d_fa, nspec));
   PTC_TRY(alloc(&S.d_fb, nspec));
-  PTC_TRY(alloc(&S.d_cell, (size_t)c->nx * (c->ny + 2) * c->nz));
-  PTC_TRY(alloc(&S.d_px, (size_t)c->ny * S.nch * (c->nx / 2 + 1)));
-  PTC_TRY(alloc(&S.d_pz, (size_t)2 * c->ny * c->nz));
+  PTC_TRY(alloc(&S.d_toprow, (size_t)3 * c->nx * c->nz));
+  PTC_TRY(alloc(&S.d_top, (size_t)S.pitch * c->nz));
+  PTC_TRY(alloc(&S.d_px, (size_t)spec_products(kSet) * c->ny * S.nch * (c->nx / 2 + 1)));
+  int ns, nt, nseg;
+  sums_shape(c->nx / 2, &ns, &nt, &nseg);
+  PTC_TRY(alloc(&S.d_pz, (size_t)2 * spec_products(kSet) * c->ny * c->nz * nseg));
   // the symbol of the cell-centre interpolation of ux, kx = 0..nx/2
   const int h = c->nx / 2;
   const double ic[4] = {c->geo.ic1, c->geo.ic2, c->geo.ic3, c->geo.ic4};
@@ -379,7 +393,8 @@ void spectra_free(ptc_ctx *c) {
   release(S.d_iy2d);
   release(S.d_fa);
   release(S.d_fb);
-  release(S.d_cell);
+  release(S.d_toprow);
+  release(S.d_top);
   release(S.d_px);
   release(S.d_pz);
   release(S.d_hx);
@@ -426,7 +441,7 @@ int spectra_init(ptc_ctx *c, int clc1d, int jlcs, int clc2d, int ny2d, const int
 }
 
 // One sample (src/m_FlowCase.f90:430-805), in the order that keeps two
-// spectra live: the cell-centre uy in fb throughout, each other field in fa.
+// spectra live: uy in fb throughout, each other field in fa.
 int spectra_sample(ptc_ctx *c, const double *ux, const double *uy, const double *uz, const double *p,
                    const double *sc) {
   SpectraState &S = c->spec;
@@ -439,41 +454,37 @@ int spectra_sample(ptc_ctx *c, const double *ux, const double *uy, const double 
   PTC_TRY(ensure_work(c));
   const int ny = c->ny;
   const double crf = (double)c->nx * (double)c->nz * c->prm.ucrf;  // ux + uCRF moves F(0, 0) only
-  SpecPair P{};
-  // cell-centre uy -> fb
-  PTC_TRY(cell_uy(c, uy));
-  PTC_TRY(forward(c, S.d_cell, S.d_fb));
+  // uy -> fb: energy (2); 2-D (2, the face mirror)
+  SpecIn P{};
+  PTC_TRY(forward(c, uy, S.d_fb));
+  PTC_TRY(forward_top(c, uy));
+  P.a = S.d_fb;
+  if (S.on1d) PTC_TRY(spec_1d(c, P, kEnergy, 2));
+  if (S.on2d) PTC_TRY(spec_2d(c, S.d_fb, S.d_fb, 2, 2, 1.0));
   // ux -> fa: energy (1), linear coherence (7, 8), co-spectra with the
   // cell-centre uy of ux + uCRF (5) and of the cell-centre ux (6, H(kx) fa);
   // 2-D: ux (1) and the cell-centre co-spectrum (5, IsSymmetry = .false.: rCoe = -1)
   PTC_TRY(forward(c, ux, S.d_fa));
   if (S.on1d) {
-    P = SpecPair{S.d_fa, S.d_fa, crf, crf, 0, 0, 0, 0, nullptr};
-    PTC_TRY(spec_1d(c, P, true, 0, 1, 1));
     // :473-489: rows 1..nyc/2 against jForLCS, a channel's upper rows against nyc+1-jForLCS
     const bool ch = c->prm.flow_type == 1;
-    P = SpecPair{S.d_fa, S.d_fa, crf, crf, 1, S.jlcs - 1, ch ? ny - S.jlcs : S.jlcs - 1, ch ? ny / 2 : ny, nullptr};
-    PTC_TRY(spec_1d(c, P, false, 1, 7, 8));
-    P = SpecPair{S.d_fa, S.d_fb, crf, 0.0, 0, 0, 0, 0, nullptr};
-    PTC_TRY(spec_1d(c, P, false, 0, 5, 5));
-    P = SpecPair{S.d_fa, S.d_fb, crf, 0.0, 0, 0, 0, 0, S.d_hx};
-    PTC_TRY(spec_1d(c, P, false, 0, 6, 6));
+    P = SpecIn{S.d_fa, S.d_fb, S.d_top, S.d_hx, crf, S.jlcs - 1, ch ? ny - S.jlcs : S.jlcs - 1, ch ? ny / 2 : ny};
+    PTC_TRY(spec_1d(c, P, kSet, 0));
   }
   if (S.on2d) {
     PTC_TRY(spec_2d(c, S.d_fa, S.d_fa, 1, 1, 1.0));
-    PTC_TRY(spec_2d(c, S.d_fa, S.d_fb, 5, 1, -1.0, S.d_hx, crf));
+    PTC_TRY(spec_2d(c, S.d_fa, S.d_fb, 5, 1, -1.0, S.d_top, S.d_hx, crf));
   }
-  // uy (2-D: the face mirror), uz, p, scalar
-  const double *rest[4] = {uy, uz, p, sc};
-  const int m1[4] = {2, 3, 4, 9}, m2[4] = {2, 3, 4, 6};
-  for (int q = 0; q < 4; ++q) {
-    if (q == 3 && !c->prm.scalar) break;
+  // uz, p, scalar
+  const double *rest[3] = {uz, p, sc};
+  const int m1[3] = {3, 4, 9}, m2[3] = {3, 4, 6};
+  for (int q = 0; q < 3; ++q) {
+    if (q == 2 && !c->prm.scalar) break;
     PTC_TRY(forward(c, rest[q], S.d_fa));
-    if (S.on1d) {
-      P = SpecPair{S.d_fa, S.d_fa, 0.0, 0.0, 0, 0, 0, 0, nullptr};
-      PTC_TRY(spec_1d(c, P, true, 0, m1[q], m1[q]));
-    }
-    if (S.on2d) PTC_TRY(spec_2d(c, S.d_fa, S.d_fa, m2[q], q == 0 ? 2 : 1, 1.0));
+    P = SpecIn{};
+    P.a = S.d_fa;
+    if (S.on1d) PTC_TRY(spec_1d(c, P, kEnergy, m1[q]));
+    if (S.on2d) PTC_TRY(spec_2d(c, S.d_fa, S.d_fa, m2[q], 1, 1.0));
   }
   ++S.nspectime;
   return PTC_OK;

@@ -1486,32 +1486,6 @@ int get_device_scalar(ptc_ctx *c, int slot, double *out) {
 namespace ptc {
 
 // ---- clcStat (src/m_FlowCase.f90:283-413) ----------------------------------
-// Sums NS values over a wavefront: each of six exchanges sends half of the values
-// a lane still holds to the lane that keeps them, so NS values cost about NS
-// exchanges instead of 6 NS.  On return lane l holds the sum of value *idx in
-// v[0] (*idx = -1: none).  Fixed order.
-template <int NS, int N, int MASK>
-__device__ __forceinline__ void wave_sums_step(double (&v)[NS], int lane, int &base, int &count) {
-  constexpr int H = (N + 1) / 2;
-  const bool up = lane & MASK;
-#pragma unroll
-  for (int q = 0; q < H; ++q) {
-    const double hi = q + H < N ? v[q + H] : 0.0;
-    const double send = up ? v[q] : hi, keep = up ? hi : v[q];
-    v[q] = keep + __shfl_xor(send, MASK);
-  }
-  base += up ? H : 0;
-  count = up ? count - H : min(count, H);
-  if constexpr (MASK > 1) wave_sums_step<NS, H, MASK / 2>(v, lane, base, count);
-}
-template <int NS>
-__device__ __forceinline__ void wave_sums(double (&v)[NS], int lane, int *idx) {
-  static_assert(NS <= 64, "one value per lane at the end");
-  int base = 0, count = NS;
-  wave_sums_step<NS, NS, 32>(v, lane, base, count);
-  *idx = count > 0 ? base : -1;
-}
-
 // The reference's SumVec terms of rows j = 1..ny, marching z as k_rhs_rows does: a
 // workgroup owns rows of x (one thread per column; rows longer than 256 points go
 // in segments of 252 with two wrapped halo columns on either side) and marches
