@@ -124,15 +124,12 @@ __global__ void __launch_bounds__(MAXT) k_fft_x_fwd(const double *__restrict__ s
   extern __shared__ double2 lds[];
   const int h = L.n, G = L.threads;
   const int l = threadIdx.x / G, g = threadIdx.x - l * G;
-  const long long nlines = (long long)ny * nz;
   const int tt = tj * tk;
   const int wb = DIV ? xcd_run((int)blockIdx.x, (int)gridDim.x, tt >= nl ? 2 * tt / nl : 1) : (int)blockIdx.x;
-  const long long q = (long long)wb * nl + l;
-  const bool live = l < nl && q < nlines;
-  const long long qq = live ? q : 0;
-  const long long tq = DIV ? qq / tt : 0, wq = qq - tq * tt, ntk = nz / tk;
-  const long long jl = DIV ? (tq / ntk) * tj + wq / tk : qq % ny;
-  const long long k = DIV ? (tq % ntk) * tk + wq % tk : qq / ny;
+  const unsigned q = (unsigned)wb * nl + l;
+  const bool live = l < nl && q < (unsigned)ny * nz;
+  const LineAt at0 = line_at<DIV>(live ? q : 0, ny, nz, tj, tk);
+  const long long jl = at0.j, k = at0.k;
   double2 *ls = lds + (l < nl ? l : 0) * (rt_pad(h - 1, pad) + 2);
   const double2 *row = reinterpret_cast<const double2 *>(src + rowlen * (jl + 1 + (long long)(ny + 2) * k));
   double dmax = 0.0;
@@ -189,17 +186,17 @@ __global__ void __launch_bounds__(MAXT) k_fft_x_inv(const double2 *__restrict__ 
   extern __shared__ double2 lds[];
   const int h = L.n, G = L.threads;
   const int l = threadIdx.x / G, g = threadIdx.x - l * G;
-  const long long q = (long long)blockIdx.x * nl + l;
-  const bool live = l < nl && q < (long long)ny * nz;
-  const long long qq = live ? q : 0;
-  const long long jl = qq % ny, k = qq / ny;
+  const unsigned q = blockIdx.x * nl + l;
+  const bool live = l < nl && q < (unsigned)ny * nz;
+  const LineAt at0 = line_at<false>(live ? q : 0, ny, nz, 1, 1);
+  const long long jl = at0.j, k = at0.k;
   double2 *ls = lds + (l < nl ? l : 0) * (rt_pad(h, pad) + 1);
   auto at = [&](int m) { return ls[rt_pad(m, pad)]; };
   auto put = [&](int m, double2 v) { ls[rt_pad(m, pad)] = v; };
   if (live) {
     // the line's h+1 values go through LDS once; eight loads in flight
     // (indices past h repeat element h)
-    const double2 *in = spec + qq * pitch;
+    const double2 *in = spec + (jl + (long long)ny * k) * pitch;
     for (int m0 = g; m0 <= h; m0 += 8 * G) {
       double2 v[8];
 #pragma unroll

@@ -307,7 +307,15 @@ constexpr int f2_x_min_waves() {
 // needs (three waves per SIMD at most).
 template <int N, int SRC>
 constexpr int f2_xfwd_min_waves() {
-  return SRC == 2 ? ((N == 2304 || N == 4608) ? 3 : 1) : f2_x_min_waves<N>();
+  return SRC >= 2 ? ((N == 2304 || N == 4608) ? 3 : 1) : f2_x_min_waves<N>();
+}
+// Lines of one plane column in the column form of the residual (kXResCol), or
+// 0 where the length has none: a workgroup's lines in groups of K consecutive
+// planes of one row, N * lines a multiple of K * 256.
+template <int N>
+constexpr int f2_res_lines() {
+  constexpr int L = f2_threads<N>() <= 256 ? 256 / f2_threads<N>() : 1;
+  return f2_xblock<N>() == 256 && L * f2_threads<N>() == 256 ? (L % 8 == 0 ? 8 : (L == 4 ? 4 : 0)) : 0;
 }
 
 // ---- x forward: nlpb real rows of length 2N -> half spectra ---------------
@@ -319,13 +327,105 @@ constexpr int f2_xfwd_min_waves() {
 // SRC = kXRes: the rows are the refinement's FP64 residual f - L phi, in
 // k_residual's operand order; each workgroup writes the sum of phi over its
 // lines of row j = 1 to rs.psum[blockIdx.x].
-constexpr int kXPlain = 0, kXDiv = 1, kXRes = 2;
+// SRC = kXResCol: the same residual, formed by columns.  The direct form loads
+// fifteen pairs per pair of points (five of its own row, six planes, two rows,
+// f), 16 GB through L1 at 1024x256x512; here a thread forms one pair m of K
+// consecutive planes, whose K + 6 planes it loads once, and reads the row
+// neighbours from the lines' LDS: 5.5 (K = 4) or 4.75 (K = 8) loads a pair.
+// 1022 -> 780 us there with FP32 spectra (2.1 GB in, 0.5 GB out; the shape of
+// the tiles and f's caching hint move it by under 1 %: it waits on its two
+// rounds of loads, at three waves per SIMD).
+// Needs tk a multiple of K, so that no group of K lines leaves its row.
+constexpr int kXPlain = 0, kXDiv = 1, kXRes = 2, kXResCol = 3;
+
+// The residual of a workgroup's lines q0 .. q0+L-1 into their LDS rows (the
+// column form).  Each thread takes the columns threadIdx.x + 256 c: pair m of
+// the K planes of one group of lines.  All the planes of its columns are in
+// flight at once, then the rows above and below and f, one column after the
+// other; edge rows load their own row for the missing one (the Neumann
+// condition), so no load sits behind a branch.
+template <int N, int K, bool STREAM>
+__device__ __forceinline__ void res_columns(double2 *sh, const ResSrc &rs, const Geo &geo, int ny, int nz,
+                                            long long rowlen, int j0, unsigned q0, unsigned nlines, int tj, int tk,
+                                            double &psum) {
+  constexpr double st0 = -1460.0 / 576.0, st1 = 783.0 / 576.0, st2 = -54.0 / 576.0, st3 = 1.0 / 576.0;
+  constexpr int L = 256 / f2_threads<N>();
+  constexpr int NC = N * (L / K) / 256;  // columns per thread
+  static_assert(NC * 256 == N * (L / K), "whole columns");
+  constexpr int PN = xpadded<N>();
+  const long long pl = rowlen * (ny + 2);
+  double2 z[NC][K + 6];
+  long long base[NC];  // offset of the group's first line
+  int mc[NC], gc[NC], jc[NC];
+  bool ok[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int col = (int)threadIdx.x + 256 * c;
+    mc[c] = col % N;
+    gc[c] = col / N;
+    const unsigned q = q0 + gc[c] * K;
+    ok[c] = q < nlines;
+    const LineAt at = line_at<true>(ok[c] ? q : 0, 1, nz, tj, tk);
+    const int jl = j0 + at.j, k = at.k;
+    jc[c] = jl + 1;
+    base[c] = rowlen * (jl + 1 + (long long)(ny + 2) * k);
+#pragma unroll
+    for (int s = 0; s < K + 6; ++s) {
+      int kk = k - 3 + s;
+      kk = kk < 0 ? kk + nz : (kk >= nz ? kk - nz : kk);
+      z[c][s] = reinterpret_cast<const double2 *>(rs.phi + base[c] + (kk - k) * pl)[mc[c]];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int i = 0; i < K; ++i) sh[(gc[c] * K + i) * PN + xpad<N>(mc[c])] = z[c][3 + i];
+  __syncthreads();
+  double2 r[NC][K];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int m = mc[c], j = jc[c];
+    const double am = geo.met[M_AM2PH * geo.nyh + j], ac = geo.met[M_AC2PH * geo.nyh + j],
+                 ap = geo.met[M_AP2PH * geo.nyh + j];
+    const int m1 = m - 1 < 0 ? m - 1 + N : m - 1, m2 = m - 2 < 0 ? m - 2 + N : m - 2;
+    const int p1 = m + 1 >= N ? m + 1 - N : m + 1, p2 = m + 2 >= N ? m + 2 - N : m + 2;
+    const int om = j > 1 ? m - N : m, op = j < ny ? m + N : m;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const double2 *pr = reinterpret_cast<const double2 *>(rs.phi + base[c] + i * pl);
+      const double2 ym = pr[om], yp = pr[op];
+      const double2 fv = f2::ld2x<STREAM>(reinterpret_cast<const double2 *>(rs.f + base[c] + i * pl)[m]);
+      const double2 *row = sh + (gc[c] * K + i) * PN;
+      const double2 a1 = row[xpad<N>(m1)], b1 = row[xpad<N>(p1)];
+      const double a0 = row[xpad<N>(m2)].y, b2 = row[xpad<N>(p2)].x;
+      const double2 *zz = z[c] + i;  // planes k-3 .. k+3
+      const double2 c0 = zz[3];
+      const double lx0 = st0 * c0.x + st1 * (a1.y + c0.y) + st2 * (a1.x + b1.x) + st3 * (a0 + b1.y);
+      const double lx1 = st0 * c0.y + st1 * (c0.x + b1.x) + st2 * (a1.y + b1.y) + st3 * (a1.x + b2);
+      const double lz0 = st0 * c0.x + st1 * (zz[2].x + zz[4].x) + st2 * (zz[1].x + zz[5].x) + st3 * (zz[0].x + zz[6].x);
+      const double lz1 = st0 * c0.y + st1 * (zz[2].y + zz[4].y) + st2 * (zz[1].y + zz[5].y) + st3 * (zz[0].y + zz[6].y);
+      const double lap0 = rs.rdx2 * lx0 + rs.rdz2 * lz0 + (am * ym.x + ac * c0.x + ap * yp.x);
+      const double lap1 = rs.rdx2 * lx1 + rs.rdz2 * lz1 + (am * ym.y + ac * c0.y + ap * yp.y);
+      if (j == 1 && ok[c]) {
+        psum += c0.x;
+        psum += c0.y;
+      }
+      r[c][i] = make_double2(fv.x - lap0, fv.y - lap1);
+    }
+  }
+  __syncthreads();  // every thread has read its neighbours
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int i = 0; i < K; ++i) sh[(gc[c] * K + i) * PN + xpad<N>(mc[c])] = r[c][i];
+}
+
 template <int N, typename S, bool STREAM, int SRC>
 __global__ void __launch_bounds__(f2_xblock<N>(), (f2_xfwd_min_waves<N, SRC>())) k2_fft_x_fwd(const double *__restrict__ src, S *__restrict__ spec,
                                                     const double2 *__restrict__ tw, const double2 *__restrict__ wx,
                                                     int ny, int nz, int j0, int nj, int pitch, long long rowlen,
                                                     DivSrc dv, ResSrc rs, Geo geo, int tj, int tk) {
-  constexpr bool DIV = SRC == kXDiv, RES = SRC == kXRes, NBR = DIV || RES;
+  constexpr bool DIV = SRC == kXDiv, COL = SRC == kXResCol, RES = SRC == kXRes || COL, NBR = DIV || RES;
   constexpr int G = f2_threads<N>();
   constexpr int L = (256 / G) > 0 ? 256 / G : 1;
   constexpr int PN = xpadded<N>();
@@ -338,16 +438,13 @@ __global__ void __launch_bounds__(f2_xblock<N>(), (f2_xfwd_min_waves<N, SRC>()))
   // tile, the tiles k fastest) and runs of two tiles' workgroups go to one XCD
   // (xcd_run), so the neighbouring lines that re-read a row, in j or in k, do
   // so through the same L2.
-  const long long nlines = (long long)nj * nz;
+  const unsigned nlines = (unsigned)nj * nz;
   const int tt = tj * tk;
-  const long long wb = NBR ? (long long)xcd_run((int)blockIdx.x, (int)gridDim.x, tt >= L ? 2 * tt / L : 1)
-                           : (long long)blockIdx.x;
-  const long long q = wb * L + l;
+  const unsigned wb = NBR ? (unsigned)xcd_run((int)blockIdx.x, (int)gridDim.x, tt >= L ? 2 * tt / L : 1) : blockIdx.x;
+  const unsigned q = wb * L + l;
   const bool live = l < L && q < nlines;
-  const long long qq = live ? q : 0;
-  const long long tq = qq / tt, wq = qq - tq * tt, ntk = nz / tk;
-  const long long jl = NBR ? j0 + (tq / ntk) * tj + wq / tk : j0 + qq % nj;
-  const long long k = NBR ? (tq % ntk) * tk + wq % tk : qq / nj;
+  const LineAt at = line_at<NBR>(live ? q : 0, nj, nz, tj, tk);
+  const long long jl = j0 + at.j, k = at.k;
   const long long sq = jl + (long long)ny * k;  // spectral row S[k][jl]
   const double2 *row = reinterpret_cast<const double2 *>(src + rowlen * (jl + 1 + (long long)(ny + 2) * k));
   double2 *ls = sh + (l < L ? l : 0) * PN;
@@ -400,7 +497,13 @@ __global__ void __launch_bounds__(f2_xblock<N>(), (f2_xfwd_min_waves<N, SRC>()))
   };
   auto lds = [&](int m) -> double2 & { return ls[xpad<N>(m)]; };
   auto store_lds = [&](int m, double2 v) { ls[xpad<N>(m)] = v; };
-  f2::run_fft<N, G, false>(g, tw, load0, lds, store_lds);
+  if constexpr (COL) {
+    res_columns<N, f2_res_lines<N>(), STREAM>(sh, rs, geo, ny, nz, rowlen, j0, wb * L, nlines, tj, tk, psum);
+    __syncthreads();
+    f2::run_fft<N, G, false, true>(g, tw, lds, lds, store_lds);
+  } else {
+    f2::run_fft<N, G, false>(g, tw, load0, lds, store_lds);
+  }
   __syncthreads();
   if (live) x_untangle_store<N, G, STREAM>(g, ls, wx, spec + sq * pitch, pitch);
   if constexpr (DIV) {
@@ -441,11 +544,10 @@ __global__ void __launch_bounds__(f2_xblock<N>(), f2_x_min_waves<N>())
   constexpr int PN = xpadded<N>();
   __shared__ double2 sh[L * PN];
   const int l = threadIdx.x / G, g = threadIdx.x - l * G;
-  const long long nlines = (long long)nj * nz;
-  const long long q = (long long)blockIdx.x * L + l;
-  const bool live = l < L && q < nlines;
-  const long long qq = live ? q : 0;
-  const long long jl = j0 + qq % nj, k = qq / nj;
+  const unsigned q = blockIdx.x * L + l;
+  const bool live = l < L && q < (unsigned)nj * nz;
+  const LineAt at = line_at<false>(live ? q : 0, nj, nz, 1, 1);
+  const long long jl = j0 + at.j, k = at.k;
   const S *in = spec + (jl + (long long)ny * k) * pitch;
   double2 *ls = sh + (l < L ? l : 0) * PN;
   // The re-tangle of element m needs X_m and X_{N-m}: the line's N+1 values
@@ -527,15 +629,15 @@ __global__ void __launch_bounds__(f2_xblock<N>()) k2p_fft_x_fwd(const double *__
   constexpr int BPT0 = f2::stage_bpt<N, 0, G>();
   __shared__ double2 sh[L * PN];
   const int l = threadIdx.x / G, g = threadIdx.x - l * G;
-  const long long nlines = (long long)nj * nz;
+  const unsigned nlines = (unsigned)nj * nz;
   const long long ngroups = (nlines + L - 1) / L;
   double2 *ls = sh + l * PN;
   // line l of group grp: rows j fastest; sq = its spectral row
   auto line = [&](long long grp, bool &live, long long &sq) {
-    const long long q = grp * L + l;
+    const unsigned q = (unsigned)grp * L + l;
     live = q < nlines;
-    const long long qq = live ? q : 0;
-    const long long jl = j0 + qq % nj, k = qq / nj;
+    const LineAt at = line_at<false>(live ? q : 0, nj, nz, 1, 1);
+    const long long jl = j0 + at.j, k = at.k;
     sq = jl + (long long)ny * k;
     return reinterpret_cast<const double2 *>(src + rowlen * (jl + 1 + (long long)(ny + 2) * k));
   };
@@ -598,16 +700,16 @@ __global__ void __launch_bounds__(f2_xblock<N>()) k2p_fft_x_inv(const S *__restr
   constexpr int NT = N / G + 1;
   __shared__ double2 sh[L * PN];
   const int l = threadIdx.x / G, g = threadIdx.x - l * G;
-  const long long nlines = (long long)nj * nz;
+  const unsigned nlines = (unsigned)nj * nz;
   const long long ngroups = (nlines + L - 1) / L;
   double2 *ls = sh + l * PN;
   const double sh0 = ACC ? shift[0] : 0.0;
   auto coords = [&](long long grp, bool &live, long long &jl, long long &k) {
-    const long long q = grp * L + l;
+    const unsigned q = (unsigned)grp * L + l;
     live = q < nlines;
-    const long long qq = live ? q : 0;
-    jl = j0 + qq % nj;
-    k = qq / nj;
+    const LineAt at = line_at<false>(live ? q : 0, nj, nz, 1, 1);
+    jl = j0 + at.j;
+    k = at.k;
   };
   // the line's N+1 spectral values (indices past N repeat element N)
   auto fetch = [&](long long grp, double2 (&v)[NT]) {
@@ -793,6 +895,22 @@ static void x_fwd_launch(ptc_ctx *c, const double *src, S *spec, int j0, int nj,
                      tj, tk);
 }
 
+// the residual by columns where the length has the form and the tiles of
+// lines hold whole groups of its planes, else pair by pair
+template <int N, bool STREAM>
+static void x_res_launch(ptc_ctx *c, float2 *spec, int j0, int nj, const ResSrc &res) {
+  constexpr int K = f2_res_lines<N>();
+  if constexpr (K > 0) {
+    int tj, tk;
+    line_tile(nj, c->nz, &tj, &tk);
+    if (tk % K == 0) {
+      x_fwd_launch<N, float2, STREAM, kXResCol>(c, nullptr, spec, j0, nj, DivSrc{}, res);
+      return;
+    }
+  }
+  x_fwd_launch<N, float2, STREAM, kXRes>(c, nullptr, spec, j0, nj, DivSrc{}, res);
+}
+
 template <int N>
 static int x_fwd_t(ptc_ctx *c, const double *src, void *spec, int j0, int nj, bool f64, const DivSrc *div,
                    const ResSrc *res) {
@@ -804,10 +922,9 @@ static int x_fwd_t(ptc_ctx *c, const double *src, void *spec, int j0, int nj, bo
     else x_fwd_launch<N, double2, false, kXDiv>(c, src, (double2 *)spec, j0, nj, *div);
   } else if (res) {
     // the one-shot kernel forms the residual, whatever the plan's x form
-    if (f32 && c->pp.stream) x_fwd_launch<N, float2, true, kXRes>(c, src, (float2 *)spec, j0, nj, none, *res);
-    else if (f32) x_fwd_launch<N, float2, false, kXRes>(c, src, (float2 *)spec, j0, nj, none, *res);
-    else if (c->pp.stream) x_fwd_launch<N, double2, true, kXRes>(c, src, (double2 *)spec, j0, nj, none, *res);
-    else x_fwd_launch<N, double2, false, kXRes>(c, src, (double2 *)spec, j0, nj, none, *res);
+    PTC_CHECK(f32, PTC_E_STATE, "the residual-forming x pass belongs to the FP32-storage refinement");
+    if (c->pp.stream) x_res_launch<N, true>(c, (float2 *)spec, j0, nj, *res);
+    else x_res_launch<N, false>(c, (float2 *)spec, j0, nj, *res);
   } else if (c->pp.persist_x) {
     if constexpr (has_px(N)) {
       if (f32 && c->pp.stream) px_fwd_launch<N, float2, true>(c, src, (float2 *)spec, j0, nj);
