@@ -146,63 +146,83 @@ __device__ __forceinline__ void chunk_backsub(V (&f)[MM], const double (&A)[MM],
   f[0] = xs;
 }
 
-// Reduced system of 2P rows per line (row 2p: first row of chunk p, row 2p+1:
-// its last row), unit diagonal, solved by parallel cyclic reduction: at step d
-// every row eliminates its neighbours q-d and q+d, so after ceil(log2(2P))
-// steps each row stands alone.  Rows outside the system act as decoupled
-// identity rows.  The rows live in LDS, double-buffered ([2][2P][LPB] for
-// each of a, c, f): a step reads one buffer and writes the other, so it needs
-// one barrier and holds nothing in registers across steps.  The reference
+// Reduced system of 2P rows per line (chunk p's first row, its last row), unit
+// diagonal.  The first rows go first: each last row substitutes its chunk's
+// first row and the next chunk's, which leaves P rows in the last values alone,
+// solved by parallel cyclic reduction: at step d every row eliminates its
+// neighbours p-d and p+d, so after ceil(log2 P) steps each row stands alone;
+// the first value then follows from its row.  (All 2P rows through the
+// reduction took one more step and twice the rows a step: the y pass of
+// 1024x256x512 with FP32 spectra 343 us, now 253; a solve of 128x96x128 51.8,
+// now 49.8; errors against the oracle as before or smaller.)  Rows outside the
+// system act as decoupled identity rows.  They live in LDS, double-buffered ([2][P][LPB]
+// for each of a, c, f): a step reads one buffer and writes the other, so it
+// needs one barrier and holds nothing in registers across steps.  The reference
 // solves the same reduced system by Thomas (InverseTridiagonal_reduce,
 // src/m_Poisson.f90:1045-1071); cyclic reduction lets every chunk's lane take
 // part instead of one wavefront.
-template <int LPB, typename V>
-__device__ __forceinline__ void pcr_row(int q, int d, int n2, int lane, const double *RA, const double *RC,
-                                        const V *RF, double *WA, double *WC, V *WF) {
-  const int o = q * LPB + lane;
-  const double a = RA[o], c = RC[o];
-  V f = RF[o];
-  double am = 0.0, cm = 0.0, ap = 0.0, cp = 0.0;
-  V fm = vzero(f), fp = vzero(f);
-  if (q - d >= 0) {
-    am = RA[o - d * LPB];
-    cm = RC[o - d * LPB];
-    fm = RF[o - d * LPB];
-  }
-  if (q + d < n2) {
-    ap = RA[o + d * LPB];
-    cp = RC[o + d * LPB];
-    fp = RF[o + d * LPB];
-  }
-  // a x_{q-d} + x_q + c x_{q+d} = f, with rows q-d and q+d substituted
+
+// the row a x_m + x + c x_p = f with the rows am .. + x_m + cm x = fm and
+// ap x + x_p + cp .. = fp substituted (in and out)
+template <typename V>
+__device__ __forceinline__ void pcr_substitute(double &a, double &c, V &f, double am, double cm, V fm, double ap,
+                                               double cp, V fp) {
   const double inv = 1.0 / (1.0 - a * cm - c * ap);
-  WF[o] = vscale(inv, vsub(vsub(f, vscale(a, fm)), vscale(c, fp)));
-  WA[o] = -inv * a * am;
-  WC[o] = -inv * c * cp;
+  f = vscale(inv, vsub(vsub(f, vscale(a, fm)), vscale(c, fp)));
+  a = -inv * a * am;
+  c = -inv * c * cp;
 }
 
 template <int LPB, typename V>
 __device__ __forceinline__ void solve_reduced(double aS, double cS, V fS, double aE, double cE, V fE, int P, int p,
                                               int lane, double *RA, double *RC, V *RF, V &xs, V &xe) {
-  const int n2 = 2 * P, q0 = 2 * p, q1 = 2 * p + 1;
-  const int half = n2 * LPB;  // second buffer
-  RA[q0 * LPB + lane] = aS;
-  RC[q0 * LPB + lane] = cS;
-  RF[q0 * LPB + lane] = fS;
-  RA[q1 * LPB + lane] = aE;
-  RC[q1 * LPB + lane] = cE;
-  RF[q1 * LPB + lane] = fE;
-  int in = 0;
-  for (int d = 1; d < n2; d *= 2) {
-    __syncthreads();
-    const int out = half - in;
-    pcr_row<LPB>(q0, d, n2, lane, RA + in, RC + in, RF + in, RA + out, RC + out, RF + out);
-    pcr_row<LPB>(q1, d, n2, lane, RA + in, RC + in, RF + in, RA + out, RC + out, RF + out);
-    in = out;
+  const int half = P * LPB, o = p * LPB + lane;  // half: the second buffer
+  RA[o] = aS;
+  RC[o] = cS;
+  RF[o] = fS;
+  __syncthreads();
+  double a = aE, c = cE;
+  V f = fE;
+  {
+    double ap = 0.0, cp = 0.0;
+    V fp = vzero(f);
+    if (p + 1 < P) {
+      ap = RA[o + LPB];
+      cp = RC[o + LPB];
+      fp = RF[o + LPB];
+    }
+    pcr_substitute(a, c, f, aS, cS, fS, ap, cp, fp);
   }
-  // each thread reads back only the rows it wrote itself
-  xs = RF[in + q0 * LPB + lane];
-  xe = RF[in + q1 * LPB + lane];
+  int in = half;
+  RA[in + o] = a;
+  RC[in + o] = c;
+  RF[in + o] = f;
+  for (int d = 1; d < P; d *= 2) {
+    __syncthreads();
+    double am = 0.0, cm = 0.0, ap = 0.0, cp = 0.0;
+    V fm = vzero(f), fp = vzero(f);
+    if (p - d >= 0) {
+      am = RA[in + o - d * LPB];
+      cm = RC[in + o - d * LPB];
+      fm = RF[in + o - d * LPB];
+    }
+    if (p + d < P) {
+      ap = RA[in + o + d * LPB];
+      cp = RC[in + o + d * LPB];
+      fp = RF[in + o + d * LPB];
+    }
+    pcr_substitute(a, c, f, am, cm, fm, ap, cp, fp);
+    in = half - in;
+    if (2 * d < P) {
+      RA[in + o] = a;
+      RC[in + o] = c;
+    }
+    RF[in + o] = f;
+  }
+  __syncthreads();
+  xe = f;
+  const V xm = p > 0 ? RF[in + o - LPB] : vzero(f);
+  xs = vsub(vsub(fS, vscale(aS, xm)), vscale(cS, xe));
 }
 
 // chunk index of a thread; with 64 lines per block a chunk is one wavefront
@@ -235,8 +255,8 @@ __global__ void __launch_bounds__(1024) k_tri_poisson_split(S *__restrict__ spec
                                                            int P) {
   extern __shared__ double smem[];
   double *RA = smem;
-  double *RC = RA + 4 * P * LPB;
-  double *RF = RC + 4 * P * LPB;
+  double *RC = RA + 2 * P * LPB;
+  double *RF = RC + 2 * P * LPB;
   const int lane = threadIdx.x % LPB;
   const int p = chunk_of_thread<LPB>();
   const int kx = blockIdx.x * (LPB / 2) + lane / 2, kz = blockIdx.y;
@@ -330,7 +350,7 @@ __global__ void __launch_bounds__(512) k_tri_poisson_lds(S *__restrict__ spec, c
   double aS, cS, aE, cE, fS, fE, xs, xe;
   chunk_reduce<MM>(f, A, C, s, getc, aS, cS, fS, aE, cE, fE);
   __syncthreads();  // every chunk has left the tile: it becomes the reduction's buffers
-  double *RA = tile, *RC = RA + 4 * P * LL, *RF = RC + 4 * P * LL;
+  double *RA = tile, *RC = RA + 2 * P * LL, *RF = RC + 2 * P * LL;
   solve_reduced<LL>(aS, cS, fS, aE, cE, fE, P, p, line, RA, RC, RF, xs, xe);
   chunk_backsub<MM>(f, A, C, xs, xe);
   __syncthreads();  // the reduction's buffers are read: back to the tile
@@ -394,10 +414,10 @@ __device__ __forceinline__ void cst(float2 &d, double2 v) {
 }
 
 // LDS of the complex-line kernel in doubles: the three coefficient rows
-// (padded to 16 bytes) and a, c, f (f complex) of 2P reduced rows x LC lines,
+// (padded to 16 bytes) and a, c, f (f complex) of P reduced rows x LC lines,
 // double-buffered
 constexpr size_t tri_cplx_lds_doubles(int nyh, int P, int LC) {
-  return (size_t)((3 * nyh + 1) / 2 * 2) + (size_t)16 * P * LC;
+  return (size_t)((3 * nyh + 1) / 2 * 2) + (size_t)8 * P * LC;
 }
 
 // chunks of 12 or more complex rows need more than 128 VGPRs: their
@@ -412,8 +432,8 @@ __global__ void __launch_bounds__(tri_cplx_cap(MM)) k_tri_poisson_cplx(S *__rest
   extern __shared__ double smem[];
   double *mA = smem, *mC = mA + nyh, *mP = mC + nyh;
   double *RA = smem + (3 * nyh + 1) / 2 * 2;  // 16-byte aligned
-  double *RC = RA + 4 * P * LC;
-  double2 *RF = reinterpret_cast<double2 *>(RC + 4 * P * LC);
+  double *RC = RA + 2 * P * LC;
+  double2 *RF = reinterpret_cast<double2 *>(RC + 2 * P * LC);
   const int t = threadIdx.x;
   const int lane = t % LC, p = t / LC;
   const int kx = blockIdx.x * LC + lane, kz = blockIdx.y;
@@ -503,7 +523,7 @@ __global__ void __launch_bounds__(256) k_tri_poisson_thomas(double2 *__restrict_
 // The matrix I - beta L_y of a job is the same for every line (i, k).  Its
 // chunk elimination factors, the reduced rows and the coefficients of every
 // cyclic-reduction step are formed by k_cn_factor (one workgroup per job,
-// the same arithmetic chunk_reduce and pcr_row apply to the coefficients;
+// the same arithmetic chunk_reduce and solve_reduced apply to the coefficients;
 // once per launch, or once per beta for the tables a step keeps), and the
 // solve reads them as wave-uniform scalars: it
 // keeps only the right-hand side and the old u in registers and does no
@@ -579,7 +599,8 @@ __global__ void __launch_bounds__(64) k_cn_factor(CnJobs jobs, const double *__r
     sa[0][2 * t + 1] = aE;
     sc[0][2 * t + 1] = cE;
   }
-  // pcr_row on the coefficients: each step's (a, c, inv) of every reduced row
+  // pcr_substitute on the coefficients: each step's (a, c, inv) of every reduced
+  // row (of the chunks' first rows the solve reads step 0's a and c)
   int in = 0, l = 0;
   for (int d = 1; d < n2; d *= 2, ++l) {
     __syncthreads();
@@ -644,7 +665,7 @@ __device__ double flow_fold_shift(const FlowFold &ff, double *red) {
 template <int MM, int LPB>
 __global__ void __launch_bounds__(tri_cn_block_cap<MM>()) k_tri_cn_fac(CnJobs jobs, const double *__restrict__ fac,
                                                                      int nx, int ny, int P, FlowFold ff) {
-  extern __shared__ double smem[];  // f of the 2P reduced rows x LPB lines, double-buffered
+  extern __shared__ double smem[];  // f of the P reduced rows x LPB lines, double-buffered
   double *RF = smem;
   const CnJob &J = jobs.j[blockIdx.z];
   const double *__restrict__ T = fac + (long long)J.tab * kCnFacStride;
@@ -695,27 +716,31 @@ __global__ void __launch_bounds__(tri_cn_block_cap<MM>()) k_tri_cn_fac(CnJobs jo
 #pragma unroll
   for (int r = MM - 3; r >= 1; --r) g = f[r] - T[X.C(s + r)] * g;
   const double fS = T[X.r0(p)] * (f[0] - T[X.c0(p)] * g);
-  // reduced rows by cyclic reduction (pcr_row with the step coefficients read)
-  const int n2 = 2 * P, q0 = 2 * p, q1 = 2 * p + 1, half = n2 * LPB;
-  RF[q0 * LPB + lane] = fS;
-  RF[q1 * LPB + lane] = fE;
-  int in = 0, l = 0;
-  for (int d = 1; d < n2; d *= 2, ++l) {
-    __syncthreads();
-    const int out = half - in;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int q = h ? q1 : q0;
-      const int o = q * LPB + lane;
-      const double *e = T + X.pcr(l, q);
-      const double fc = RF[in + o];
-      const double fm = q - d >= 0 ? RF[in + o - d * LPB] : 0.0;
-      const double fp = q + d < n2 ? RF[in + o + d * LPB] : 0.0;
-      RF[out + o] = e[2] * ((fc - e[0] * fm) - e[1] * fp);
-    }
-    in = out;
+  // reduced rows (solve_reduced with the step coefficients read)
+  const int half = P * LPB, o = p * LPB + lane;
+  RF[o] = fS;
+  __syncthreads();
+  double xe;
+  {
+    const double *e = T + X.pcr(0, 2 * p + 1);
+    const double fp = p + 1 < P ? RF[o + LPB] : 0.0;
+    xe = e[2] * ((fE - e[0] * fS) - e[1] * fp);
   }
-  const double xs = RF[in + q0 * LPB + lane], xe = RF[in + q1 * LPB + lane];
+  int in = half, l = 1;
+  RF[in + o] = xe;
+  for (int d = 1; d < P; d *= 2, ++l) {
+    __syncthreads();
+    const double *e = T + X.pcr(l, 2 * p + 1);
+    const double fm = p - d >= 0 ? RF[in + o - d * LPB] : 0.0;
+    const double fp = p + d < P ? RF[in + o + d * LPB] : 0.0;
+    xe = e[2] * ((xe - e[0] * fm) - e[1] * fp);
+    in = half - in;
+    RF[in + o] = xe;
+  }
+  __syncthreads();
+  const double xm = p > 0 ? RF[in + o - LPB] : 0.0;
+  const double *eS = T + X.pcr(0, 2 * p);
+  const double xs = (fS - eS[0] * xm) - eS[1] * xe;
   // back substitution (chunk_backsub)
   f[MM - 1] = xe;
 #pragma unroll
@@ -774,7 +799,7 @@ static int tri_choose(int ny, size_t lds_limit, int mm_req, int lpb_req, const T
       if (lpb * P > shapes[q].cap) continue;
       if (2 * P * lpb > 1 << 16) continue;
       if (pass == 0 && (P * mm - ny) * 8 > ny) continue;  // prefer little padding
-      const size_t lds = (size_t)4 * P * lpb * 24;  // a, c, f of the reduced rows, two buffers
+      const size_t lds = (size_t)2 * P * lpb * 24;  // a, c, f of the reduced rows, two buffers
       if (lds > lds_limit) continue;
       *P_out = P;
       *mm_out = mm;
@@ -790,7 +815,7 @@ static int tri_choose(int ny, size_t lds_limit, int mm_req, int lpb_req, const T
 // LDS-staged Poisson kernel: LL lines per workgroup, P * LL <= 512 threads,
 // LDS = row coefficients + max(tile, reduction buffers)
 size_t tri_lds_bytes(int ny, int P, int ll) {
-  const size_t tile = (size_t)ny * (ll + 1), red = (size_t)12 * P * ll;
+  const size_t tile = (size_t)ny * (ll + 1), red = (size_t)6 * P * ll;
   return sizeof(double) * (3 * (size_t)(ny + 2) + std::max(tile, red));
 }
 
@@ -913,7 +938,7 @@ int launch_tri_poisson(ptc_ctx *c, void *spec) {
   const int nP = P.tri_chunks, lpb = P.tri_lpb;
   // lpb lanes per block = lpb/2 complex lines
   dim3 grid((unsigned)((2 * (P.h + 1) + lpb - 1) / lpb), (unsigned)c->nz);
-  const size_t lds = (size_t)4 * nP * lpb * 24;
+  const size_t lds = (size_t)2 * nP * lpb * 24;
 #define PTC_CASE(MM, LPB)                                                                                     \
   if (P.tri_mmax == MM && lpb == LPB) {                                                                       \
     if (f32)                                                                                                  \
@@ -968,7 +993,7 @@ static int launch_cn(ptc_ctx *c, const CnJobs &jobs, bool factor, bool solve, co
   PTC_TRY(tri_plan(c->ny, c->lds_limit, false, 0, 0, &nP, &mmax, &lpb));
   PTC_CHECK(nP * mmax <= 256 && 2 * nP <= 64, PTC_E_STATE, "Crank-Nicolson chunk plan outside the factor table");
   dim3 grid((unsigned)((c->nx + lpb - 1) / lpb), (unsigned)c->nz, (unsigned)jobs.n);
-  const size_t lds = sizeof(double) * 2 * (size_t)(2 * nP) * lpb;
+  const size_t lds = sizeof(double) * 2 * (size_t)nP * lpb;
 #define PTC_CN(MM, LPB)                                                                                        \
   if (mmax == MM && lpb == LPB) {                                                                              \
     if (factor) {                                                                                              \
