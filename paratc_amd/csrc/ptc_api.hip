@@ -329,7 +329,7 @@ int channel_step(ptc_ctx *c, double *mon) {
     if (poisson_div_fusable(c)) {
       const DivSrc dv{ux, uy, uz, 1.0 / c->pmAlpha, c->d_red};
       PTC_TRY(poisson_solve_div(c, dv, hl, true));
-      if (ns == c->iadvance) PTC_TRY(launch_divmax(c, (int)fft_x_fwd_blocks(c, c->ny)));
+      if (ns == c->iadvance) PTC_TRY(launch_divmax(c, (int)fft_x_div_blocks(c, c->ny)));
     } else {
       PTC_TRY(launch_prsrc(c, ux, uy, uz, a1, nullptr, ns == c->iadvance));
       PTC_TRY(poisson_solve(c, a1, hl, true));

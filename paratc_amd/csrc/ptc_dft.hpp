@@ -285,54 +285,6 @@ struct Dft<16, INV> {
 
 }  // namespace f2
 
-// The pair of points (2m, 2m+1) of row j = jl + 1, plane k of the Poisson
-// source, formed from the velocities as clcPrSrc does (src/m_TScheme.f90:48-77):
-// sudtal times the divergence with the 4th-order staggered x and z differences
-// and the 2nd-order y difference, in k_prsrc's operand order.  n2 = nx / 2 pairs
-// in a row of rowlen = nx values; dmax: running max |divergence|.
-__device__ __forceinline__ double2 div_pair(const DivSrc &dv, const Geo &geo, int n2, int ny, int nz,
-                                            long long rowlen, long long jl, long long k, int m, double &dmax) {
-  const long long rj = rowlen * (jl + 1 + (long long)(ny + 2) * k);
-  const double2 *uxr = reinterpret_cast<const double2 *>(dv.ux + rj);
-  const double2 *uyr = reinterpret_cast<const double2 *>(dv.uy + rj);
-  const int mm = m > 0 ? m - 1 : n2 - 1, mp = m + 1 < n2 ? m + 1 : 0;
-  const double2 a = uxr[mm], b = uxr[m], cc = uxr[mp];
-  const double2 y0 = uyr[m], y1 = uyr[m + n2];
-  const long long pl = rowlen * (ny + 2);
-  double2 z[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    long long kk = k - 1 + s;
-    kk = kk < 0 ? kk + nz : (kk >= nz ? kk - nz : kk);
-    z[s] = reinterpret_cast<const double2 *>(dv.uz + rj + (kk - k) * pl)[m];
-  }
-  const double rdyp = geo.met[M_RDYP * geo.nyh + jl + 1];
-  const double dudx0 = geo.dxc1 * a.y + geo.dxc2 * b.x + geo.dxc3 * b.y + geo.dxc4 * cc.x;
-  const double dudx1 = geo.dxc1 * b.x + geo.dxc2 * b.y + geo.dxc3 * cc.x + geo.dxc4 * cc.y;
-  const double dvdy0 = (y1.x - y0.x) * rdyp, dvdy1 = (y1.y - y0.y) * rdyp;
-  const double dwdz0 = geo.dzc1 * z[0].x + geo.dzc2 * z[1].x + geo.dzc3 * z[2].x + geo.dzc4 * z[3].x;
-  const double dwdz1 = geo.dzc1 * z[0].y + geo.dzc2 * z[1].y + geo.dzc3 * z[2].y + geo.dzc4 * z[3].y;
-  const double r0 = dudx0 + dvdy0 + dwdz0, r1 = dudx1 + dvdy1 + dwdz1;
-  dmax = fmax(dmax, fmax(fabs(r0), fabs(r1)));
-  return make_double2(dv.sudtal * r0, dv.sudtal * r1);
-}
-
-// the maximum of v over a workgroup by a fixed-order tree in red (one value
-// per thread), after a barrier that ends earlier uses of that memory
-__device__ __forceinline__ double block_max_tree(double v, double *red) {
-  const int t = threadIdx.x;
-  __syncthreads();
-  red[t] = v;
-  __syncthreads();
-  for (int n = blockDim.x; n > 1;) {
-    const int h = (n + 1) / 2;
-    if (t < n - h) red[t] = fmax(red[t], red[t + h]);
-    __syncthreads();
-    n = h;
-  }
-  return red[0];
-}
-
 // Row j and plane k (both 0-based, j within the pass's nj rows) of line q of an
 // x pass, in 32 bits: a line is at least 128 bytes, so fewer than 2^31 of them
 // fit the device.  (In 64 bits each lane made up to four long divisions before
@@ -353,6 +305,109 @@ __device__ __forceinline__ LineAt line_at(unsigned q, unsigned nj, unsigned nz, 
     const unsigned k = q / nj;
     return LineAt{(int)(q - k * nj), (int)k};
   }
+}
+
+// The values of the Poisson source at the pair of points (2m, 2m+1), formed as
+// clcPrSrc does (src/m_TScheme.f90:48-77): sudtal times the divergence
+// (point_div).  a, b, c: the pairs m-1, m, m+1 of ux; y0, y1: the
+// pair of uy in rows j, j+1; z[0..3]: that of uz in planes k-1 .. k+2; dmax: running
+// max |divergence|.
+__device__ __forceinline__ double2 div_value(const DivSrc &dv, const Geo &geo, double rdyp, double2 a, double2 b,
+                                             double2 c, double2 y0, double2 y1, const double2 *z, double &dmax) {
+  const double r0 = point_div(geo, rdyp, a.y, b.x, b.y, c.x, y0.x, y1.x, z[0].x, z[1].x, z[2].x, z[3].x);
+  const double r1 = point_div(geo, rdyp, b.x, b.y, c.x, c.y, y0.y, y1.y, z[0].y, z[1].y, z[2].y, z[3].y);
+  dmax = fmax(dmax, fmax(fabs(r0), fabs(r1)));
+  return make_double2(dv.sudtal * r0, dv.sudtal * r1);
+}
+
+// One pair of a row, straight into a transform's first stage (rows of which a
+// workgroup holds one).  n2 = nx / 2 pairs in a row of rowlen = nx values.
+__device__ __forceinline__ double2 div_pair(const DivSrc &dv, const Geo &geo, int n2, int ny, int nz,
+                                            long long rowlen, long long jl, long long k, int m, double &dmax) {
+  const long long rj = rowlen * (jl + 1 + (long long)(ny + 2) * k);
+  const double2 *uxr = reinterpret_cast<const double2 *>(dv.ux + rj);
+  const double2 *uyr = reinterpret_cast<const double2 *>(dv.uy + rj);
+  const int mm = m > 0 ? m - 1 : n2 - 1, mp = m + 1 < n2 ? m + 1 : 0;
+  const double2 a = uxr[mm], b = uxr[m], cc = uxr[mp];
+  const double2 y0 = uyr[m], y1 = uyr[m + n2];
+  const long long pl = rowlen * (ny + 2);
+  double2 z[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    long long kk = k - 1 + s;
+    kk = kk < 0 ? kk + nz : (kk >= nz ? kk - nz : kk);
+    z[s] = reinterpret_cast<const double2 *>(dv.uz + rj + (kk - k) * pl)[m];
+  }
+  const double rdyp = geo.met[M_RDYP * geo.nyh + jl + 1];
+  return div_value(dv, geo, rdyp, a, b, cc, y0, y1, z, dmax);
+}
+
+// The rows of a workgroup's nl lines (q0 ...) into its LDS lines, by columns: a
+// thread forms one pair m of K consecutive planes at a time, whose K + 3 planes
+// of uz it loads once, and consecutive lanes take consecutive pairs of a row.
+// (Formed in the transform's first stage, each pair loaded all nine of its
+// values, four to sixteen lanes to a row.)  Lines come in groups of K planes,
+// nzp = nz rounded up to whole groups of them, nlines = rows times nzp: the
+// lines of planes past nz are zero and never stored.  slot(l, m): element m of
+// the workgroup's line l.
+template <int K, class Slot>
+__device__ __forceinline__ void div_columns(const DivSrc &dv, const Geo &geo, int n2, int ny, int nz, int nzp,
+                                            long long rowlen, int j0, unsigned nlines, int tj, int tk, unsigned q0,
+                                            int nl, int nthr, const Slot &slot, double &dmax) {
+  const long long pl = rowlen * (ny + 2);
+  const int ncol = n2 * (nl / K);
+  for (int c = threadIdx.x; c < ncol; c += nthr) {
+    const int grp = (unsigned)c / (unsigned)n2, m = c - grp * n2;
+    const unsigned q = q0 + grp * K;
+    const bool on = q < nlines;
+    const LineAt at = line_at<true>(on ? q : 0, 1, nzp, tj, tk);
+    const int j = j0 + at.j + 1, k = at.k;
+    const long long rj = rowlen * (j + (long long)(ny + 2) * k);
+    const int mm = m > 0 ? m - 1 : n2 - 1, mp = m + 1 < n2 ? m + 1 : 0;
+    double2 z[K + 3], a[K], b[K], cc[K], y0[K], y1[K];
+#pragma unroll
+    for (int s = 0; s < K + 3; ++s) {
+      int kk = min(k - 1 + s, nz + 1);
+      kk = kk < 0 ? kk + nz : (kk >= nz ? kk - nz : kk);
+      z[s] = reinterpret_cast<const double2 *>(dv.uz + rj + (kk - k) * pl)[m];
+    }
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const long long o = rj + (min(k + i, nz - 1) - k) * pl;
+      const double2 *uxr = reinterpret_cast<const double2 *>(dv.ux + o);
+      const double2 *uyr = reinterpret_cast<const double2 *>(dv.uy + o);
+      a[i] = uxr[mm];
+      b[i] = uxr[m];
+      cc[i] = uxr[mp];
+      y0[i] = uyr[m];
+      y1[i] = uyr[m + n2];
+    }
+    const double rdyp = geo.met[M_RDYP * geo.nyh + j];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      double d = 0.0;
+      const double2 v = div_value(dv, geo, rdyp, a[i], b[i], cc[i], y0[i], y1[i], z + i, d);
+      const bool live = on && k + i < nz;
+      if (live) dmax = fmax(dmax, d);
+      slot(grp * K + i, m) = live ? v : make_double2(0.0, 0.0);
+    }
+  }
+}
+
+// the maximum of v over a workgroup by a fixed-order tree in red (one value
+// per thread), after a barrier that ends earlier uses of that memory
+__device__ __forceinline__ double block_max_tree(double v, double *red) {
+  const int t = threadIdx.x;
+  __syncthreads();
+  red[t] = v;
+  __syncthreads();
+  for (int n = blockDim.x; n > 1;) {
+    const int h = (n + 1) / 2;
+    if (t < n - h) red[t] = fmax(red[t], red[t + h]);
+    __syncthreads();
+    n = h;
+  }
+  return red[0];
 }
 
 // line tiles of the neighbour-reading x passes: the largest of 8, 4, 2, 1 rows

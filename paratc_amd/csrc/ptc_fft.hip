@@ -350,9 +350,9 @@ int fft_z_tile(const FftLen &L, size_t lds_cap, int most) {
   return T;
 }
 
-long long fft_x_fwd_blocks(const ptc_ctx *c, int nj) {
+long long fft_x_div_blocks(const ptc_ctx *c, int nj) {
   const PoissonPlan &P = c->pp;
-  if (P.x_fast || !P.ready) return fft2_x_fwd_blocks(c, nj);
+  if (P.x_fast || !P.ready) return fft2_x_div_blocks(c, nj);
   return ((long long)nj * c->nz + P.x_lines - 1) / P.x_lines;
 }
 
@@ -361,8 +361,9 @@ static void x_fwd_rt(ptc_ctx *c, const double *src, double2 *spec, const DivSrc 
   PoissonPlan &P = c->pp;
   int tj = 1, tk = 1;
   if (DIV) line_tile(c->ny, c->nz, &tj, &tk);
-  hipLaunchKernelGGL((k_fft_x_fwd<DIV, STREAM, MAXT, RMAX>), dim3((unsigned)fft_x_fwd_blocks(c, c->ny)), dim3(P.x_threads),
-                     P.x_lds, c->stream, src, spec, P.fx, P.d_wx, c->ny, c->nz, P.x_lines, P.x_pad, P.pitch,
+  const long long nlines = (long long)c->ny * c->nz;
+  hipLaunchKernelGGL((k_fft_x_fwd<DIV, STREAM, MAXT, RMAX>), dim3((unsigned)((nlines + P.x_lines - 1) / P.x_lines)),
+                     dim3(P.x_threads), P.x_lds, c->stream, src, spec, P.fx, P.d_wx, c->ny, c->nz, P.x_lines, P.x_pad, P.pitch,
                      (long long)c->nx, dv, c->geo, tj, tk);
 }
 

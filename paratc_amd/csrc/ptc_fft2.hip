@@ -229,10 +229,20 @@ constexpr int f2_threads() {
   return N / (f2::plan_rmax(N) > 8 ? 8 : f2::plan_rmax(N));
 }
 
-// x-pass workgroup: 256 threads (several lines) or one line of G > 256 threads
+// x-pass workgroup: about 64 threads for rows of up to 256 points, about 256 for
+// longer ones (several lines each), or one line of G > 256 threads.  Short rows
+// belong to small grids, whose few hundred workgroups of 256 threads leave CUs
+// idle and fill the last round unevenly: RK substep 64x48x64 58.1 -> 55.1 us,
+// 96x64x96 84.5 -> 83.0, 128x48x64 68.0 -> 66.4, 192x64x96 126.7 -> 123.8,
+// 128x96x128 and 192x128x192 the same; rows of 512 points 1239 -> 1235 at 128.
+template <int N>
+constexpr int f2_xbase() {
+  return N <= 128 ? 64 : 256;
+}
+// its threads at most
 template <int N>
 constexpr int f2_xblock() {
-  return f2_threads<N>() > 256 ? f2_threads<N>() : 256;
+  return f2_threads<N>() > f2_xbase<N>() ? f2_threads<N>() : f2_xbase<N>();
 }
 
 // LDS layout of an x-pass line: one padding value after every 8 (bank
@@ -305,28 +315,44 @@ constexpr int f2_x_min_waves() {
 // The residual-forming form holds twenty more loads per point pair: held to
 // those bounds it spills 96-188 bytes per lane, so it takes the registers it
 // needs (three waves per SIMD at most).
+// The divergence by columns of 512- and 1024-point rows is held to 128 VGPRs (it
+// takes 130 left alone).
 template <int N, int SRC>
 constexpr int f2_xfwd_min_waves() {
-  return SRC >= 2 ? ((N == 2304 || N == 4608) ? 3 : 1) : f2_x_min_waves<N>();
+  return SRC >= 2 ? ((N == 2304 || N == 4608) ? 3 : 1) : (SRC == 1 && N >= 256 && N <= 512 ? 4 : f2_x_min_waves<N>());
+}
+// Planes a thread takes at a time where the divergence is formed by columns
+// (1: pair by pair), and the lines of a workgroup then, whole groups of them.
+template <int N>
+constexpr int f2_div_planes() {
+  constexpr int L = f2_threads<N>() <= f2_xbase<N>() ? f2_xbase<N>() / f2_threads<N>() : 1;
+  return L >= 4 ? 4 : (L >= 2 ? 2 : 1);
+}
+template <int N>
+constexpr int f2_div_lines() {
+  constexpr int L = f2_threads<N>() <= f2_xbase<N>() ? f2_xbase<N>() / f2_threads<N>() : 1;
+  return L / f2_div_planes<N>() * f2_div_planes<N>();
 }
 // Lines of one plane column in the column form of the residual (kXResCol), or
 // 0 where the length has none: a workgroup's lines in groups of K consecutive
 // planes of one row, N * lines a multiple of K * 256.
 template <int N>
 constexpr int f2_res_lines() {
-  constexpr int L = f2_threads<N>() <= 256 ? 256 / f2_threads<N>() : 1;
-  return f2_xblock<N>() == 256 && L * f2_threads<N>() == 256 ? (L % 8 == 0 ? 8 : (L == 4 ? 4 : 0)) : 0;
+  constexpr int L = f2_threads<N>() <= f2_xbase<N>() ? f2_xbase<N>() / f2_threads<N>() : 1;
+  return L * f2_threads<N>() == f2_xbase<N>() ? (L % 8 == 0 ? 8 : (L == 4 ? 4 : 0)) : 0;
 }
 
 // ---- x forward: nlpb real rows of length 2N -> half spectra ---------------
 // SRC = kXDiv: the rows are not read from src but formed from the velocities,
-// as clcPrSrc does (src/m_TScheme.f90:48-77): sudtal times the divergence of
-// (ux, uy, uz) with the 4th-order staggered x and z differences and the 2nd-
-// order y difference, in k_prsrc's operand order.  Each workgroup then writes
+// as clcPrSrc does (div_value), by columns of planes where a workgroup holds two
+// lines or more (f2_div_planes), else pair by pair.  Each workgroup then writes
 // the maximum |divergence| over its rows to dv.part[blockIdx.x].
 // SRC = kXRes: the rows are the refinement's FP64 residual f - L phi, in
 // k_residual's operand order; each workgroup writes the sum of phi over its
 // lines of row j = 1 to rs.psum[blockIdx.x].
+// By columns and in workgroups of 64 threads (rows of up to 256 points) the RK
+// substep of 64x48x64 took 55.1 us against 59.2, 192x64x96 123.8 against 127.4,
+// 512x128x256 1234 against 1250; by columns alone 58.1, 126.6 and 1240.
 // SRC = kXResCol: the same residual, formed by columns.  The direct form loads
 // fifteen pairs per pair of points (five of its own row, six planes, two rows,
 // f), 16 GB through L1 at 1024x256x512; here a thread forms one pair m of K
@@ -349,9 +375,9 @@ __device__ __forceinline__ void res_columns(double2 *sh, const ResSrc &rs, const
                                             long long rowlen, int j0, unsigned q0, unsigned nlines, int tj, int tk,
                                             double &psum) {
   constexpr double st0 = -1460.0 / 576.0, st1 = 783.0 / 576.0, st2 = -54.0 / 576.0, st3 = 1.0 / 576.0;
-  constexpr int L = 256 / f2_threads<N>();
-  constexpr int NC = N * (L / K) / 256;  // columns per thread
-  static_assert(NC * 256 == N * (L / K), "whole columns");
+  constexpr int T = f2_xbase<N>(), L = T / f2_threads<N>();
+  constexpr int NC = N * (L / K) / T;  // columns per thread
+  static_assert(NC * T == N * (L / K), "whole columns");
   constexpr int PN = xpadded<N>();
   const long long pl = rowlen * (ny + 2);
   double2 z[NC][K + 6];
@@ -360,7 +386,7 @@ __device__ __forceinline__ void res_columns(double2 *sh, const ResSrc &rs, const
   bool ok[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int col = (int)threadIdx.x + 256 * c;
+    const int col = (int)threadIdx.x + T * c;
     mc[c] = col % N;
     gc[c] = col / N;
     const unsigned q = q0 + gc[c] * K;
@@ -427,7 +453,8 @@ __global__ void __launch_bounds__(f2_xblock<N>(), (f2_xfwd_min_waves<N, SRC>()))
                                                     DivSrc dv, ResSrc rs, Geo geo, int tj, int tk) {
   constexpr bool DIV = SRC == kXDiv, COL = SRC == kXResCol, RES = SRC == kXRes || COL, NBR = DIV || RES;
   constexpr int G = f2_threads<N>();
-  constexpr int L = (256 / G) > 0 ? 256 / G : 1;
+  constexpr int DK = DIV ? f2_div_planes<N>() : 1;
+  constexpr int L = DIV ? f2_div_lines<N>() : ((f2_xbase<N>() / G) > 0 ? f2_xbase<N>() / G : 1);
   constexpr int PN = xpadded<N>();
   __shared__ double2 sh[L * PN];
   const int l = threadIdx.x / G, g = threadIdx.x - l * G;
@@ -438,12 +465,13 @@ __global__ void __launch_bounds__(f2_xblock<N>(), (f2_xfwd_min_waves<N, SRC>()))
   // tile, the tiles k fastest) and runs of two tiles' workgroups go to one XCD
   // (xcd_run), so the neighbouring lines that re-read a row, in j or in k, do
   // so through the same L2.
-  const unsigned nlines = (unsigned)nj * nz;
+  const unsigned nzp = DK > 1 ? (nz + DK - 1) / DK * DK : nz;  // whole groups of planes
+  const unsigned nlines = (unsigned)nj * nzp;
   const int tt = tj * tk;
   const unsigned wb = NBR ? (unsigned)xcd_run((int)blockIdx.x, (int)gridDim.x, tt >= L ? 2 * tt / L : 1) : blockIdx.x;
   const unsigned q = wb * L + l;
-  const bool live = l < L && q < nlines;
-  const LineAt at = line_at<NBR>(live ? q : 0, nj, nz, tj, tk);
+  const LineAt at = line_at<NBR>(l < L && q < nlines ? q : 0, nj, nzp, tj, tk);
+  const bool live = l < L && q < nlines && (DK == 1 || at.k < nz);
   const long long jl = j0 + at.j, k = at.k;
   const long long sq = jl + (long long)ny * k;  // spectral row S[k][jl]
   const double2 *row = reinterpret_cast<const double2 *>(src + rowlen * (jl + 1 + (long long)(ny + 2) * k));
@@ -501,6 +529,11 @@ __global__ void __launch_bounds__(f2_xblock<N>(), (f2_xfwd_min_waves<N, SRC>()))
     res_columns<N, f2_res_lines<N>(), STREAM>(sh, rs, geo, ny, nz, rowlen, j0, wb * L, nlines, tj, tk, psum);
     __syncthreads();
     f2::run_fft<N, G, false, true>(g, tw, lds, lds, store_lds);
+  } else if constexpr (DK > 1) {
+    div_columns<DK>(dv, geo, N, ny, nz, (int)nzp, rowlen, j0, nlines, tj, tk, wb * L, L, f2_xblock<N>(),
+                    [&](int line, int m) -> double2 & { return sh[line * PN + xpad<N>(m)]; }, dmax);
+    __syncthreads();
+    f2::run_fft<N, G, false, true>(g, tw, lds, lds, store_lds);
   } else {
     f2::run_fft<N, G, false>(g, tw, load0, lds, store_lds);
   }
@@ -540,7 +573,7 @@ __global__ void __launch_bounds__(f2_xblock<N>(), f2_x_min_waves<N>())
                                                     int ny, int nz, int j0, int nj, int pitch, long long rowlen,
                                                     double scale, const double *__restrict__ shift, int ghost) {
   constexpr int G = f2_threads<N>();
-  constexpr int L = (256 / G) > 0 ? 256 / G : 1;
+  constexpr int L = (f2_xbase<N>() / G) > 0 ? f2_xbase<N>() / G : 1;
   constexpr int PN = xpadded<N>();
   __shared__ double2 sh[L * PN];
   const int l = threadIdx.x / G, g = threadIdx.x - l * G;
@@ -622,7 +655,7 @@ __global__ void __launch_bounds__(f2_xblock<N>()) k2p_fft_x_fwd(const double *__
                                                      const double2 *__restrict__ tw, const double2 *__restrict__ wx,
                                                      int ny, int nz, int j0, int nj, int pitch, long long rowlen) {
   constexpr int G = f2_threads<N>();
-  constexpr int L = (256 / G) > 0 ? 256 / G : 1;
+  constexpr int L = (f2_xbase<N>() / G) > 0 ? f2_xbase<N>() / G : 1;
   constexpr int PN = xpadded<N>();
   constexpr int R0 = f2::make_plan(N).r[0];
   constexpr int NB0 = N / R0;
@@ -695,7 +728,7 @@ __global__ void __launch_bounds__(f2_xblock<N>()) k2p_fft_x_inv(const S *__restr
                                                      int ny, int nz, int j0, int nj, int pitch, long long rowlen,
                                                      double scale, const double *__restrict__ shift, int ghost) {
   constexpr int G = f2_threads<N>();
-  constexpr int L = (256 / G) > 0 ? 256 / G : 1;
+  constexpr int L = (f2_xbase<N>() / G) > 0 ? f2_xbase<N>() / G : 1;
   constexpr int PN = xpadded<N>();
   constexpr int NT = N / G + 1;
   __shared__ double2 sh[L * PN];
@@ -846,7 +879,7 @@ static unsigned persistent_grid(const ptc_ctx *c, int per_cu, long long items) {
 template <int N, typename S, bool STREAM>
 static void px_fwd_launch(ptc_ctx *c, const double *src, S *spec, int j0, int nj) {
   constexpr int G = f2_threads<N>();
-  constexpr int L = (256 / G) > 0 ? 256 / G : 1;
+  constexpr int L = (f2_xbase<N>() / G) > 0 ? f2_xbase<N>() / G : 1;
   static const int per_cu = resident_blocks(k2p_fft_x_fwd<N, S, STREAM>, L * G);
   const long long groups = ((long long)nj * c->nz + L - 1) / L;
   hipLaunchKernelGGL((k2p_fft_x_fwd<N, S, STREAM>), dim3(persistent_grid(c, per_cu, groups)), dim3(L * G), 0,
@@ -857,7 +890,7 @@ static void px_fwd_launch(ptc_ctx *c, const double *src, S *spec, int j0, int nj
 template <int N, typename S, bool ACC, bool STREAM>
 static void px_inv_launch(ptc_ctx *c, const S *spec, double *dst, double scale, int j0, int nj, bool ghost) {
   constexpr int G = f2_threads<N>();
-  constexpr int L = (256 / G) > 0 ? 256 / G : 1;
+  constexpr int L = (f2_xbase<N>() / G) > 0 ? f2_xbase<N>() / G : 1;
   static const int per_cu = resident_blocks(k2p_fft_x_inv<N, S, ACC, STREAM>, L * G);
   const long long groups = ((long long)nj * c->nz + L - 1) / L;
   hipLaunchKernelGGL((k2p_fft_x_inv<N, S, ACC, STREAM>), dim3(persistent_grid(c, per_cu, groups)), dim3(L * G), 0,
@@ -878,19 +911,27 @@ static void pz_launch(ptc_ctx *c, S *spec, int j0, int nj) {
 template <int N>
 static long long x_fwd_blocks(long long nlines) {
   constexpr int G = f2_threads<N>();
-  constexpr int L = (256 / G) > 0 ? 256 / G : 1;
+  constexpr int L = (f2_xbase<N>() / G) > 0 ? f2_xbase<N>() / G : 1;
   return (nlines + L - 1) / L;
+}
+
+// workgroups of the divergence-forming pass
+template <int N>
+static long long x_div_blocks(int nj, int nz) {
+  constexpr int K = f2_div_planes<N>(), L = f2_div_lines<N>();
+  return ((long long)nj * ((nz + K - 1) / K * K) + L - 1) / L;
 }
 
 template <int N, typename S, bool STREAM, int SRC>
 static void x_fwd_launch(ptc_ctx *c, const double *src, S *spec, int j0, int nj, const DivSrc &dv,
                          const ResSrc &rs = ResSrc{}) {
   constexpr int G = f2_threads<N>();
-  constexpr int L = (256 / G) > 0 ? 256 / G : 1;
-  const unsigned nblk = (unsigned)x_fwd_blocks<N>((long long)nj * c->nz);
+  constexpr int L = (f2_xbase<N>() / G) > 0 ? f2_xbase<N>() / G : 1;
+  constexpr int DK = SRC == kXDiv ? f2_div_planes<N>() : 1;
+  const unsigned nblk = (unsigned)(SRC == kXDiv ? x_div_blocks<N>(nj, c->nz) : x_fwd_blocks<N>((long long)nj * c->nz));
   int tj, tk;
-  line_tile(nj, c->nz, &tj, &tk);
-  hipLaunchKernelGGL((k2_fft_x_fwd<N, S, STREAM, SRC>), dim3(nblk), dim3(L * G), 0, c->stream, src, spec,
+  line_tile(nj, (c->nz + DK - 1) / DK * DK, &tj, &tk);
+  hipLaunchKernelGGL((k2_fft_x_fwd<N, S, STREAM, SRC>), dim3(nblk), dim3(DK > 1 ? f2_xblock<N>() : L * G), 0, c->stream, src, spec,
                      c->pp.fx.tw, c->pp.d_wx, c->ny, c->nz, j0, nj, c->pp.pitch, (long long)c->nx, dv, rs, c->geo,
                      tj, tk);
 }
@@ -951,7 +992,7 @@ static int x_fwd_t(ptc_ctx *c, const double *src, void *spec, int j0, int nj, bo
 template <int N, typename S, bool ACC, bool STREAM>
 static void x_inv_launch(ptc_ctx *c, const S *spec, double *dst, double scale, int j0, int nj, bool ghost) {
   constexpr int G = f2_threads<N>();
-  constexpr int L = (256 / G) > 0 ? 256 / G : 1;
+  constexpr int L = (f2_xbase<N>() / G) > 0 ? f2_xbase<N>() / G : 1;
   const long long nlines = (long long)nj * c->nz;
   const unsigned nblk = (unsigned)((nlines + L - 1) / L);
   hipLaunchKernelGGL((k2_fft_x_inv<N, S, ACC, STREAM>), dim3(nblk), dim3(L * G), 0, c->stream, spec, dst,
@@ -1068,6 +1109,15 @@ int fft2_x_fwd(ptc_ctx *c, const double *src, void *spec, int j0, int nj, bool f
 long long fft2_x_fwd_blocks(const ptc_ctx *c, int nj) {
   switch (c->pp.h) {
 #define PTC_CASE(N) case N: return x_fwd_blocks<N>((long long)nj * c->nz);
+    PTC_X_SIZES(PTC_CASE)
+#undef PTC_CASE
+    default: return 0;
+  }
+}
+
+long long fft2_x_div_blocks(const ptc_ctx *c, int nj) {
+  switch (c->pp.h) {
+#define PTC_CASE(N) case N: return x_div_blocks<N>(nj, c->nz);
     PTC_X_SIZES(PTC_CASE)
 #undef PTC_CASE
     default: return 0;

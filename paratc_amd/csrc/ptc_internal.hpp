@@ -244,6 +244,17 @@ struct DivSrc {
   double *part;
 };
 
+// The divergence at one point: the 4th-order staggered x difference of a..d
+// (points i-1 .. i+2 of ux), the 2nd-order y difference of uy and the 4th-order z
+// difference of z0..z3, in one order of roundings for every kernel that forms
+// the Poisson source (which of two products a compiler fuses is its choice).
+__device__ __forceinline__ double point_div(const Geo &g, double rdyp, double a, double b, double c, double d,
+                                            double y0, double y1, double z0, double z1, double z2, double z3) {
+  const double dudx = fma(g.dxc4, d, fma(g.dxc3, c, fma(g.dxc2, b, g.dxc1 * a)));
+  const double dwdz = fma(g.dzc4, z3, fma(g.dzc3, z2, fma(g.dzc2, z1, g.dzc1 * z0)));
+  return fma(y1 - y0, rdyp, dudx) + dwdz;
+}
+
 // Poisson
 int poisson_build_plan(ptc_ctx *c);
 int poisson_free_plan(ptc_ctx *c);
@@ -295,8 +306,8 @@ int launch_fft_x_inv(ptc_ctx *c, const void *spec, double *dst, double scale, bo
 int launch_fft_z(ptc_ctx *c, void *spec, bool inverse, bool f64 = false);
 // the x forward pass with the Poisson source formed from the velocities (FP64 spectra)
 int launch_fft_x_fwd_div(ptc_ctx *c, const DivSrc &div, void *spec);
-// workgroups of one x forward launch over nj planes with the plan in use
-long long fft_x_fwd_blocks(const ptc_ctx *c, int nj);
+// workgroups of that pass over nj planes with the plan in use
+long long fft_x_div_blocks(const ptc_ctx *c, int nj);
 int fft_make_len(int n, FftLen *L);
 bool fft2_has_x(int h);
 bool fft2_has_z(int nz, int req, int *tile);
@@ -319,6 +330,7 @@ int fft2_x_fwd(ptc_ctx *c, const double *src, void *spec, int j0, int nj, bool f
                const DivSrc *div = nullptr, const ResSrc *res = nullptr);
 // workgroups of one specialised x forward launch over nj planes (0: no such kernel)
 long long fft2_x_fwd_blocks(const ptc_ctx *c, int nj);
+long long fft2_x_div_blocks(const ptc_ctx *c, int nj);  // and of its divergence-forming form
 // persistent prefetching forms built for this x length (nx/2) / z length and tile
 bool fft2_has_px(int h);
 bool fft2_has_pz(int nz, int tile);

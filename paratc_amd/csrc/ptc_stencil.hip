@@ -579,12 +579,9 @@ __global__ void __launch_bounds__(256) k_prsrc(Geo g, const double *__restrict__
   if (i < g.nx && j <= g.ny) {
     const Ngh N(g, i, k);
     const double rdyp = g.met[M_RDYP * g.nyh + j];
-    const double dudx = g.dxc1 * N(ux, -1, j, 0) + g.dxc2 * N(ux, 0, j, 0) + g.dxc3 * N(ux, 1, j, 0) +
-                        g.dxc4 * N(ux, 2, j, 0);
-    const double dvdy = (N(uy, 0, j + 1, 0) - N(uy, 0, j, 0)) * rdyp;
-    const double dwdz = g.dzc1 * N(uz, 0, j, -1) + g.dzc2 * N(uz, 0, j, 0) + g.dzc3 * N(uz, 0, j, 1) +
-                        g.dzc4 * N(uz, 0, j, 2);
-    const double rdiv = dudx + dvdy + dwdz;
+    const double rdiv = point_div(g, rdyp, N(ux, -1, j, 0), N(ux, 0, j, 0), N(ux, 1, j, 0), N(ux, 2, j, 0),
+                                  N(uy, 0, j, 0), N(uy, 0, j + 1, 0), N(uz, 0, j, -1), N(uz, 0, j, 0), N(uz, 0, j, 1),
+                                  N(uz, 0, j, 2));
     dm = fabs(rdiv);
     if (prsrc) prsrc[N.ii[3] + N.nxl * j + N.kk[3]] = sudtal * rdiv;
   }
@@ -1237,7 +1234,7 @@ int flow_fold(ptc_ctx *c, bool first, FlowFold *ff) {
 // reduction partials of the RHS and PrSrc kernels, allocated ahead of a
 // captured step
 int stencil_prepare(ptc_ctx *c) {
-  const int nx = (int)fft_x_fwd_blocks(c, c->ny);
+  const int nx = (int)fft_x_div_blocks(c, c->ny);
   return ensure_red(c, std::max({pt_nblocks(c), rhs_nblocks(c), nx}));
 }
 
