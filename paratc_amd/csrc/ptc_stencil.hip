@@ -613,14 +613,15 @@ struct BcArgs {
 // SetBC_and_UpdateHalo_pr (p, src/m_BC_and_Halo.f90:115-120) and
 // SetBC_and_UpdateHalo (velocities, :32-58, uy's bottom face from uy_ym) from
 // the values they have just formed: the boundary pass of the substep folded in.
-// The workgroup (64 columns x 4 rows) marches k over a chunk of planes with
-// phi's z stencil k-2 .. k+1 in registers, so each phi value is read once from
-// HBM by its own column; the x and y neighbours of phi are other lanes' rows
-// of the same plane, read through the cache.  Every load of plane k+1 is
-// issued before plane k is formed.  Runs of `run` consecutive tiles (row
-// groups fastest) go to one XCD, so a tile's edge rows are read through the L2
-// that its neighbour tiles fill (4608x140x700: 7.25 ms against 7.64 with x
-// tiles fastest).
+// The workgroup (64 or 32 pairs of columns, 256 threads) marches k over a chunk
+// of planes with phi's z stencil k-2 .. k+1 in registers, so each phi value is
+// read once from HBM by its own column; the x and y neighbours of phi are other
+// lanes' rows of the same plane, read through the cache.  Every load of plane
+// k+1 is issued before plane k is formed.  A lane takes a pair of points: 16-byte
+// accesses, and 11 loads a pair where one point a lane made 20 (RK substep
+// 256x128x192 464 -> 452 us, 128x96x128 135.6 -> 132.5, 512x128x256 1241 -> 1228).
+// Runs of `run` consecutive tiles (row groups fastest) go to one XCD, so a tile's
+// edge rows are read through the L2 that its neighbour tiles fill.
 template <bool VEL, bool PR, bool BC>
 __global__ void __launch_bounds__(256) k_vel_p_update(Geo g, const double *__restrict__ phi, double *__restrict__ ux,
                                                      double *__restrict__ uy, double *__restrict__ uz,
@@ -630,80 +631,86 @@ __global__ void __launch_bounds__(256) k_vel_p_update(Geo g, const double *__res
   const int wt = xcd_run((int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)), nwg, run);
   const int by = wt % (int)gridDim.y, bx = (wt / (int)gridDim.y) % (int)gridDim.x,
             bz = wt / (int)(gridDim.x * gridDim.y);
-  const int i = bx * 64 + threadIdx.x;
-  const int j = by * 4 + threadIdx.y + 1;
-  if (i >= g.nx || j > g.ny) return;
-  const int nx = g.nx, nz = g.nz;
+  const int nh = g.nx / 2;  // pairs of a row
+  const int m = bx * blockDim.x + threadIdx.x;
+  const int j = by * blockDim.y + threadIdx.y + 1;
+  if (m >= nh || j > g.ny) return;
+  const int nz = g.nz;
   const int k0 = bz * kc, k1 = min(k0 + kc, nz);
-  const long long pl = g.plane;
+  const long long pl = g.plane / 2;
   const int W = g.nyh;
-  const int im2 = wrapi(i - 2, nx), im1 = wrapi(i - 1, nx), ip1 = wrapi(i + 1, nx);
-  const long long rj = (long long)nx * j;
+  const int dl = (m > 0 ? m - 1 : nh - 1) - m, dr = (m + 1 < nh ? m + 1 : 0) - m;
+  const long long rj = (long long)nh * j + m;
   const double rdyc = g.met[M_RDYC * W + j];
   const double bp = -beta * g.met[M_AP2PH * W + j];
   const double bcc = -beta * g.met[M_AC2PH * W + j] + 1.0;
   const double bm = -beta * g.met[M_AM2PH * W + j];
-  auto ph = [&](int kk) { return phi[i + rj + (long long)wrapi(kk, nz) * pl]; };
+  const double2 *phi2 = reinterpret_cast<const double2 *>(phi);
+  double2 *ux2 = reinterpret_cast<double2 *>(ux), *uy2 = reinterpret_cast<double2 *>(uy),
+          *uz2 = reinterpret_cast<double2 *>(uz), *p2 = reinterpret_cast<double2 *>(p);
+  auto ph = [&](int kk) { return phi2[rj + (long long)wrapi(kk, nz) * pl]; };
   // the values of one plane that the update reads besides the phi window
   struct Plane {
-    double x, y, z, p, phm, php, xm2, xm1, xp1;
+    double2 x, y, z, p, phm, php, l;
+    double r;
   };
   auto load = [&](int k) {
     Plane q{};
-    const long long pk = (long long)k * pl, o = i + rj + pk;
-    q.phm = phi[o - nx];
-    if (PR) q.php = phi[o + nx];
+    const long long o = rj + (long long)k * pl;
+    q.phm = phi2[o - nh];
+    if (PR) q.php = phi2[o + nh];
     if (VEL) {
-      q.xm2 = phi[im2 + rj + pk];
-      q.xm1 = phi[im1 + rj + pk];
-      q.xp1 = phi[ip1 + rj + pk];
-      q.x = ux[o];
-      q.y = uy[o];
-      q.z = uz[o];
+      q.l = phi2[o + dl];
+      q.r = phi2[o + dr].x;
+      q.x = ux2[o];
+      q.y = uy2[o];
+      q.z = uz2[o];
     }
-    if (PR) q.p = p[o];
+    if (PR) q.p = p2[o];
     return q;
   };
-  double w0 = ph(k0 - 2), w1 = ph(k0 - 1), w2 = ph(k0), w3 = ph(k0 + 1);
+  double2 w0 = ph(k0 - 2), w1 = ph(k0 - 1), w2 = ph(k0), w3 = ph(k0 + 1);
   Plane cur = load(k0);
   for (int k = k0; k < k1; ++k) {
     const Plane nxt = load(k + 1 < k1 ? k + 1 : k);  // the last plane reloads its own
-    const double w4 = ph(k + 2);
-    const long long o = i + rj + (long long)k * pl;
-    double vx = 0.0, vy = 0.0, vz = 0.0, vp = 0.0;
+    const double2 w4 = ph(k + 2);
+    const long long o = rj + (long long)k * pl;
+    double2 vx{}, vy{}, vz{}, vp{};
     if (VEL) {
-      const double dpdx = g.dxc1 * cur.xm2 + g.dxc2 * cur.xm1 + g.dxc3 * w2 + g.dxc4 * cur.xp1;
-      const double dpdy = (w2 - cur.phm) * rdyc;
-      const double dpdz = g.dzc1 * w0 + g.dzc2 * w1 + g.dzc3 * w2 + g.dzc4 * w3;
-      vx = cur.x - alpha * dpdx;
-      vy = cur.y - alpha * dpdy;
-      vz = cur.z - alpha * dpdz;
-      ux[o] = vx;
-      uy[o] = vy;
-      uz[o] = vz;
+      const double dpdx0 = g.dxc1 * cur.l.x + g.dxc2 * cur.l.y + g.dxc3 * w2.x + g.dxc4 * w2.y;
+      const double dpdx1 = g.dxc1 * cur.l.y + g.dxc2 * w2.x + g.dxc3 * w2.y + g.dxc4 * cur.r;
+      const double dpdy0 = (w2.x - cur.phm.x) * rdyc, dpdy1 = (w2.y - cur.phm.y) * rdyc;
+      const double dpdz0 = g.dzc1 * w0.x + g.dzc2 * w1.x + g.dzc3 * w2.x + g.dzc4 * w3.x;
+      const double dpdz1 = g.dzc1 * w0.y + g.dzc2 * w1.y + g.dzc3 * w2.y + g.dzc4 * w3.y;
+      vx = make_double2(cur.x.x - alpha * dpdx0, cur.x.y - alpha * dpdx1);
+      vy = make_double2(cur.y.x - alpha * dpdy0, cur.y.y - alpha * dpdy1);
+      vz = make_double2(cur.z.x - alpha * dpdz0, cur.z.y - alpha * dpdz1);
+      ux2[o] = vx;
+      uy2[o] = vy;
+      uz2[o] = vz;
     }
     if (PR) {
-      vp = cur.p + bp * cur.php + bcc * w2 + bm * cur.phm;
-      p[o] = vp;
+      vp = make_double2(cur.p.x + bp * cur.php.x + bcc * w2.x + bm * cur.phm.x,
+                        cur.p.y + bp * cur.php.y + bcc * w2.y + bm * cur.phm.y);
+      p2[o] = vp;
     }
     if (BC) {
-      const long long dn = (long long)nx;  // one row
       if (j == 1) {
-        p[o - dn] = vp;
-        ux[o - dn] = b.uxb_m * 2.0 - vx;
-        uy[o] = uy_ym[i + (long long)nx * k];
-        uz[o - dn] = b.uzb_m * 2.0 - vz;
+        p2[o - nh] = vp;
+        ux2[o - nh] = make_double2(b.uxb_m * 2.0 - vx.x, b.uxb_m * 2.0 - vx.y);
+        uy2[o] = reinterpret_cast<const double2 *>(uy_ym)[m + (long long)nh * k];
+        uz2[o - nh] = make_double2(b.uzb_m * 2.0 - vz.x, b.uzb_m * 2.0 - vz.y);
       }
       if (j == g.ny) {
-        p[o + dn] = vp;
+        p2[o + nh] = vp;
         if (b.flow_type == 1) {
-          ux[o + dn] = b.uxb_p * 2.0 - vx;
-          uy[o + dn] = b.uyb_p;
-          uz[o + dn] = b.uzb_p * 2.0 - vz;
+          ux2[o + nh] = make_double2(b.uxb_p * 2.0 - vx.x, b.uxb_p * 2.0 - vx.y);
+          uy2[o + nh] = make_double2(b.uyb_p, b.uyb_p);
+          uz2[o + nh] = make_double2(b.uzb_p * 2.0 - vz.x, b.uzb_p * 2.0 - vz.y);
         } else {
-          ux[o + dn] = vx;
-          uy[o + dn] = 0.0;
-          uz[o + dn] = vz;
+          ux2[o + nh] = vx;
+          uy2[o + nh] = make_double2(0.0, 0.0);
+          uz2[o + nh] = vz;
         }
       }
     }
@@ -1284,11 +1291,9 @@ static BcArgs vel_bc_args(const ptc_ctx *c, int mode) {
   return b;
 }
 
-// z chunks of the velocity/pressure update: enough for about 96 wavefronts per
-// CU over the launch (the velocity update alone 5.34 against 5.39 ms at
-// 4608x140x700 and 0.863 against 0.892 ms at 1536x192x256 with 48), at least
-// 16 planes each (each chunk re-reads a 3-plane window prologue), shorter on
-// grids with few tiles (z_chunks)
+// z chunks of the update and the monitors: enough for about 96 wavefronts per
+// CU over the launch, at least 16 planes each (each chunk re-reads a 3-plane
+// window prologue), shorter on grids with few tiles (z_chunks)
 constexpr int kVelXcdRun = 32;
 static dim3 vel_grid(const ptc_ctx *c, int *kc) {
   const int gx = (c->nx + 63) / 64, gy = (c->ny + 3) / 4;
@@ -1298,14 +1303,31 @@ static dim3 vel_grid(const ptc_ctx *c, int *kc) {
   *kc = (c->nz + nch - 1) / nch;
   return dim3((unsigned)gx, (unsigned)gy, (unsigned)((c->nz + *kc - 1) / *kc));
 }
+// The update's blocks of 256 threads: 64 or 32 pairs wide, whichever leaves fewer
+// lanes past the row's end; 128 threads where even chunks of two planes leave
+// fewer than 1.5 workgroups per CU.  Fields are rows of an even number of
+// values, so every pair is 16-byte aligned.
+static dim3 vel2_grid(const ptc_ctx *c, int *kc, dim3 *blk) {
+  const int nh = c->nx / 2, tx = (nh + 63) / 64 * 64 * 7 > nh * 8 ? 32 : 64;
+  const int gx = (nh + tx - 1) / tx;
+  int ty = 256 / tx;
+  if (2LL * gx * ((c->ny + ty - 1) / ty) * (c->nz / 2) < 3LL * c->n_cu) ty /= 2;
+  *blk = dim3((unsigned)tx, (unsigned)ty);
+  const int gy = (c->ny + ty - 1) / ty, waves = gx * gy * (tx * ty / 64);
+  int minpl = 0;
+  const int nch = z_chunks(c->nz, (long long)gx * gy, (96 * c->n_cu + waves - 1) / waves, 16, true, c->n_cu, &minpl);
+  *kc = (c->nz + nch - 1) / nch;
+  return dim3((unsigned)gx, (unsigned)gy, (unsigned)((c->nz + *kc - 1) / *kc));
+}
 
 int launch_vel_p_update(ptc_ctx *c, const double *phi, double *ux, double *uy, double *uz, double *p) {
   const bool dv = ux && uy && uz, dp = p != nullptr;
   PTC_CHECK(dv || dp, PTC_E_ARG, "nothing to update");
   int kc = 0;
-  const dim3 grid = vel_grid(c, &kc);
+  dim3 blk;
+  const dim3 grid = vel2_grid(c, &kc, &blk);
 #define PTC_VP(V, P)                                                                                           \
-  hipLaunchKernelGGL((k_vel_p_update<V, P, false>), grid, dim3(64, 4), 0, c->stream, c->geo, phi, ux, uy, uz, p, \
+  hipLaunchKernelGGL((k_vel_p_update<V, P, false>), grid, blk, 0, c->stream, c->geo, phi, ux, uy, uz, p, \
                      c->pmAlpha, c->pmBeta, BcArgs{}, nullptr, kc, kVelXcdRun)
   if (dv && dp) PTC_VP(true, true);
   else if (dv) PTC_VP(true, false);
@@ -1318,8 +1340,9 @@ int launch_vel_p_update(ptc_ctx *c, const double *phi, double *ux, double *uy, d
 int launch_vel_p_update_bc(ptc_ctx *c, const double *phi, double *ux, double *uy, double *uz, double *p,
                            const double *uy_ym) {
   int kc = 0;
-  const dim3 grid = vel_grid(c, &kc);
-  hipLaunchKernelGGL((k_vel_p_update<true, true, true>), grid, dim3(64, 4), 0, c->stream, c->geo, phi, ux, uy, uz, p,
+  dim3 blk;
+  const dim3 grid = vel2_grid(c, &kc, &blk);
+  hipLaunchKernelGGL((k_vel_p_update<true, true, true>), grid, blk, 0, c->stream, c->geo, phi, ux, uy, uz, p,
                      c->pmAlpha, c->pmBeta, vel_bc_args(c, 5), uy_ym, kc, kVelXcdRun);
   PTC_HIP(hipGetLastError());
   return PTC_OK;
