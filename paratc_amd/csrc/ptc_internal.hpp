@@ -144,6 +144,8 @@ struct SpectraState {
   double2 *d_top = nullptr;                    // its 2-D spectrum, pitch * nz
   double *d_px = nullptr, *d_pz = nullptr;     // partial sums
   double2 *d_hx = nullptr;                     // symbol of the cell-centre interpolation of ux
+  char *h_stage[2] = {nullptr, nullptr};       // pinned halves the accumulators are read back through
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};
 };
 
 }  // namespace ptc
