@@ -905,7 +905,7 @@ int launch_visu(ptc_ctx *c, int which, const double *ux, const double *uy, const
 // The maxima of a step: CFL sum (:24-49), |divergence| (:54-81) and |ux|, |uy|,
 // |uz| (:86-110), as many of them as the instantiation asks for in one pass over
 // the velocities.  Bound by memory: 24 B per point however many are formed (one
-// pass each took 6 x 357 us a step at 1536x192x256).  As k_vel_p_update, a 64 x 4
+// pass each took 6 x 357 us a step at 1536x192x256).  A 64 x 4
 // tile marches k over a chunk of planes with uz's window in registers and the
 // next plane's loads issued before the current plane is formed.  Lanes past nx
 // and rows past ny repeat the last point, which changes no maximum.  Workgroup

@@ -9,7 +9,7 @@
 //    (src/m_Poisson.f90:497-531): afterwards row j reads
 //        x_j + a_j x_first + c_j x_last = f_j ,
 //    with the chunk's first row coupled to the previous chunk's last row.  The
-//    2P first/last rows form a tridiagonal system with unit diagonal
+//    first and last rows of the chunks form a tridiagonal system with unit diagonal
 //    (InverseTridiagonal_reduce, src/m_Poisson.f90:1045-1071) solved by
 //    cyclic reduction in LDS; every lane then reconstructs its interior rows
 //    (src/m_Poisson.f90:665-675).  One HBM read and one write per point.
