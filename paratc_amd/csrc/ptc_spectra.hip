@@ -353,7 +353,8 @@ size_t n2d(const ptc_ctx *c) { return (size_t)c->nx * c->spec.ny2d * c->nz * c->
 // work buffers sized by the current Poisson plan's spectral pitch
 int ensure_work(ptc_ctx *c) {
   SpectraState &S = c->spec;
-  if (S.d_fa && S.pitch == c->pp.pitch) return PTC_OK;
+  // (the last of them to be allocated: after a failed allocation the next call starts again)
+  if (S.d_hx && S.pitch == c->pp.pitch) return PTC_OK;
   release(S.d_fa);
   release(S.d_fb);
   release(S.d_toprow);
