@@ -386,6 +386,7 @@ void destroy(ptc_ctx *c) {
   if (c->d_visu) (void)hipFree(c->d_visu);
   if (c->d_scal) (void)hipFree(c->d_scal);
   if (c->d_cnfac) (void)hipFree(c->d_cnfac);
+  if (c->h_stat) (void)hipHostFree(c->h_stat);
   if (c->h_pinned) (void)hipHostFree(c->h_pinned);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;

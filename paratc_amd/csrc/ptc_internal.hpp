@@ -185,6 +185,7 @@ struct ptc_ctx {
   double divmax_prsrc = 0;
   ptc::PoissonPlan pp;
   double *d_stat = nullptr;  // clcStat accumulator SumStat(NCHASTAT, ny+1)
+  double *h_stat = nullptr;  // pinned: SumStat and PrGradsum as they are read
   void *d_visu = nullptr;    // dump_visu staging (visu_bytes)
   size_t visu_bytes = 0;
   int nfstime = 0;           // samples in it

@@ -49,3 +49,24 @@ def test_stat_rows_match_oracle(grid, kind):
     assert nf == 2
     assert (np.abs(one - ref) / scale).max() <= 1e-12
     assert (np.abs(two - 2 * ref) / scale).max() <= 2e-12
+
+
+@pytest.mark.parametrize("ny", [7, 31])  # 320 values and one more; 1280, a whole number of workgroups
+def test_stat_read_and_reset(ny):
+    case = E.case_channel_scalar(16, ny + 1, 8, re_b=3000.0, ws=0.02)
+    case.flow_type, case.yly, case.ny = CS.FT_HC, 1.0, ny
+    case.sections = [CS.MeshSection(1.0, ny, 1, 0, 1.7)]
+    with Solver(case) as s:
+        none, nf, pg = s.get_stat(reset=True)
+        assert not none.any() and nf == 0 and pg == 0.0
+        for q, fid in enumerate((capi.F_UX, capi.F_UY, capi.F_UZ, capi.F_PR, capi.F_SCALAR)):
+            s.upload(fid, random_halo((16, ny, 8), 70 + q))
+        s.clcStat()
+        one, nf, _ = s.get_stat()
+        kept, nf1, _ = s.get_stat(reset=True)
+        assert nf == nf1 == 1 and one[:, :ny].all() and np.array_equal(one, kept)
+        gone, nf2, pg2 = s.get_stat()
+        assert not gone.any() and nf2 == 0 and pg2 == 0.0
+        s.clcStat()
+        again, _, _ = s.get_stat()
+        assert np.array_equal(again, one)
