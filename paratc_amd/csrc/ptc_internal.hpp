@@ -379,6 +379,10 @@ struct FlowFold {
   double xnu, ubulk, ucrf, nxnz, yly, alpha, alphaC, dt;
   double *dp1ns, *prgrad;
 };
+// Lanes the flow-rate sum exchanges among in a workgroup of P chunks x lpb lanes:
+// a wavefront, or where lpb is 32 half of one (13 or 15 chunks end in half a
+// wavefront, and a lane that is not there has no defined value to exchange)
+constexpr int cn_exchange_lanes(int lpb) { return lpb < 64 ? lpb : 64; }
 constexpr int kCnMaxJobs = 4;
 // tables kept across steps: one per substep (1..3) and kind (0 u/w, 1 v, 2
 // scalar), after the kCnMaxJobs per-launch ones

@@ -630,19 +630,21 @@ __global__ void __launch_bounds__(64) k_cn_factor(CnJobs jobs, const double *__r
 
 // The constant-flow-rate shift of RhsX (src/m_TScheme.f90:269-300), in the
 // arithmetic of k_flowrate: every workgroup of the u job sums the RHS
-// kernel's partials in the same fixed order (strided per thread, across the
-// wavefront, then the wavefronts in red), so all hold the same shift; workgroup (0, 0) stores it and the
-// PrGradAver increment, as k_flowrate would.  Called by all threads.
+// kernel's partials in the same fixed order (strided per thread, across groups
+// of W lanes, then the groups in red), so all hold the same shift; workgroup (0, 0) stores it and the
+// PrGradAver increment, as k_flowrate would.  Called by all threads, whole
+// groups of W of them (cn_exchange_lanes).
+template <int W>
 __device__ double flow_fold_shift(const FlowFold &ff, double *red) {
   const int t = threadIdx.x, nt = blockDim.x;
   double acc = 0.0;
   for (int q = t; q < ff.n; q += nt) acc += ff.part[q];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-  if ((t & 63) == 0) red[t >> 6] = acc;
+  for (int off = W / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+  if (t % W == 0) red[t / W] = acc;
   __syncthreads();
   double tot = 0.0;
-  for (int w = 0; w < (nt + 63) / 64; ++w) tot += red[w];
+  for (int w = 0; w < nt / W; ++w) tot += red[w];
   __syncthreads();  // red is the solve's LDS
   double shift, inc;
   if (ff.scalar_build) {
@@ -689,7 +691,7 @@ __global__ void __launch_bounds__(tri_cn_block_cap<MM>()) k_tri_cn_fac(CnJobs jo
     uo[r] = u[o];
   }
   double sh = J.shift ? J.shift[0] : 0.0;
-  if (J.fold) sh = flow_fold_shift(ff, RF);  // uniform over the workgroup (one job)
+  if (J.fold) sh = flow_fold_shift<cn_exchange_lanes(LPB)>(ff, RF);  // uniform over the workgroup (one job)
 #pragma unroll
   for (int r = 0; r < MM; ++r) f[r] = (f[r] + sh) * ((valid && s + r < ny) ? 1.0 : 0.0);
   // du at the wall row: duy_ym, or with Update_uy_ym folded in (src/m_FlowCase.f90:112-122)

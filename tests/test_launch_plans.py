@@ -1,0 +1,43 @@
+"""Launch plans that the host forms, over all sizes they serve: what a kernel
+assumes of its workgroup and its memory holds for each (no GPU needed; the
+library's own plan functions, called from tests/launch_plans.cpp)."""
+import os
+import subprocess
+
+import pytest
+
+from paratc_amd import capi
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(capi.LIB_PATH), "csrc")
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("plans") / "launch_plans")
+    lib = os.path.dirname(os.path.abspath(capi.LIB_PATH))
+    subprocess.run(["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-host-only", "-std=c++17", "-O1", "-I", CSRC,
+                    "-I", os.path.join(HERE, "..", "include"), os.path.join(HERE, "launch_plans.cpp"), "-o", exe,
+                    "-L", lib, "-lparatc_gpu", "-Wl,-rpath," + lib], check=True)
+    out = {}
+    for line in subprocess.run([exe], capture_output=True, text=True, check=True).stdout.splitlines():
+        kind, *v = line.split()
+        out.setdefault(kind, []).append(tuple(int(q) for q in v))
+    return out
+
+
+def test_flow_rate_sum_exchanges_among_lanes_of_the_workgroup(plans):
+    """The Crank-Nicolson launch sums the flow-rate partials by lane exchanges:
+    each lane's partner is a thread of the workgroup, also where an odd number
+    of 32-lane chunks ends in half a wavefront."""
+    assert [p[0] for p in plans["cn"]] == list(range(4, 257))
+    halves = 0
+    for ny, chunks, rows, lanes, width in plans["cn"]:
+        threads = chunks * lanes
+        assert chunks * rows >= ny and width <= 64
+        halves += threads % 64 != 0
+        off = width // 2
+        while off:
+            assert all(t ^ off < threads for t in range(threads)), (ny, threads, off)
+            off //= 2
+    assert halves == 32  # ny 193-208 and 225-240
