@@ -326,20 +326,22 @@ int fft_make_len(int n, FftLen *L) {
 }
 
 // launch shape of the x passes: lines per workgroup (about 256 threads), LDS
-// padding and bytes; false if a line does not fit
-bool fft_x_shape(const FftLen &L, size_t lds_cap, int *lines, int *threads, int *pad, size_t *lds) {
+// padding and bytes; false if a line's threads or the launch's bytes do not fit.
+// Lines that pass pad_cap bytes with the padding go without it: a line holds n + 1
+// slots then (the inverse keeps X_0 .. X_n), at n = 4096 16 bytes over 64 KB.
+bool fft_x_shape(const FftLen &L, size_t pad_cap, size_t lds_limit, int *lines, int *threads, int *pad, size_t *lds) {
   if (L.threads > 1024) return false;
   *lines = std::max(1, 256 / L.threads);
   *threads = (*lines * L.threads + 63) / 64 * 64;
   *pad = 3;
   size_t slots = (size_t)L.n + L.n / 8 + 1;
-  if (sizeof(double2) * slots > lds_cap) {  // the longest lines go unpadded
+  if (sizeof(double2) * slots > pad_cap) {
     *pad = 30;
     slots = (size_t)L.n + 1;
   }
   // room for the divergence maximum's tree, one double per thread
   *lds = std::max(sizeof(double2) * slots * *lines, sizeof(double) * (size_t)*threads);
-  return sizeof(double2) * (slots - 1) <= lds_cap;
+  return *lds <= lds_limit;
 }
 
 // columns per z workgroup: the largest power of two up to `most` whose tile

@@ -28,7 +28,7 @@
 
 namespace ptc {
 
-bool fft_x_shape(const FftLen &L, size_t lds_cap, int *lines, int *threads, int *pad, size_t *lds);
+bool fft_x_shape(const FftLen &L, size_t pad_cap, size_t lds_limit, int *lines, int *threads, int *pad, size_t *lds);
 int fft_z_tile(const FftLen &L, size_t lds_cap, int most);
 int tri_plan(int ny, size_t lds_limit, bool poisson, int mm_req, int lpb_req, int *P_out, int *mm_out, int *lpb_out);
 int tri_plan_lds(int ny, size_t lds_limit, int ll, int mm_req, int *P_out, int *mm_out);
@@ -87,8 +87,8 @@ int poisson_build_plan(ptc_ctx *c) {
   P.x_fast = P.ztile_req == 0 && fft2_has_x(P.h);
   if (!P.x_fast) {
     PTC_CHECK(sizeof(double2) * (size_t)P.h <= lds_cap, PTC_E_UNSUPPORTED, "nx too large for the LDS x-FFT");
-    PTC_CHECK(fft_x_shape(P.fx, lds_cap, &P.x_lines, &P.x_threads, &P.x_pad, &P.x_lds), PTC_E_UNSUPPORTED,
-              "no x-FFT launch shape fits");
+    PTC_CHECK(fft_x_shape(P.fx, lds_cap, c->lds_limit, &P.x_lines, &P.x_threads, &P.x_pad, &P.x_lds),
+              PTC_E_UNSUPPORTED, "no x-FFT launch shape fits");
   }
 
   int zt = 0;

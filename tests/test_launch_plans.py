@@ -41,3 +41,19 @@ def test_flow_rate_sum_exchanges_among_lanes_of_the_workgroup(plans):
             assert all(t ^ off < threads for t in range(threads)), (ny, threads, off)
             off //= 2
     assert halves == 32  # ny 193-208 and 225-240
+
+
+def test_run_time_x_lines_fit_the_lds_they_ask_for(plans):
+    """Every line up to 4096 values has a launch on gfx950, and no accepted
+    launch asks for more LDS than the limit or than its kernels' last slot
+    needs: n / 8 padding slots, and one slot past the line in the inverse."""
+    seen = {}
+    for h, limit, ok, g, lines, threads, pad, nbytes in plans["x"]:
+        seen.setdefault(limit, set()).add(h)
+        if limit == 163840:
+            assert ok, h
+        if ok:
+            assert lines * g <= threads <= 1024 and nbytes <= limit, (h, nbytes)
+            line = h + (h >> pad) + 1
+            assert nbytes >= 16 * lines * line and nbytes >= 8 * threads, (h, nbytes)
+    assert seen[65536] == seen[163840] and {3375, 3675, 4096} <= seen[65536]
