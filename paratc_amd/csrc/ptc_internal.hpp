@@ -300,6 +300,7 @@ int ensure_red(ptc_ctx *c, int n);
 // the clcRhsXYZ workgroup shape in use: threads per row segment (the padded
 // row where a row is one segment), rows per workgroup, tiles per XCD run
 void rhs_shape_in_use(const ptc_ctx *c, int *seg_threads, int *rows, int *run, int *min_planes);
+size_t rhs_lds_in_use(const ptc_ctx *c);  // LDS bytes a workgroup of that shape asks for
 int poisson_residual(ptc_ctx *c, const double *src, const double *dst, double *rmax);
 int poisson_stage_times(ptc_ctx *c, float *ms5, int *nsolves);
 

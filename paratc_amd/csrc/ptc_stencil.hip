@@ -1064,8 +1064,12 @@ constexpr int kRhsXcdRun = 32;
 constexpr int kRhsMinPlanes = 16;
 constexpr size_t kRhsCachedField = size_t(256) << 20;
 struct RhsShape {
-  int tx, ty, seg, run, minpl, nseg, nyb, nch;
+  int tx, ty, seg, run, minpl, nseg, nyb, nch, lw;  // lw: LDS row width
 };
+// LDS bytes of ty rows of lw values and their two ghost rows (the kernel's last
+// sum reuses them, one double per thread)
+static size_t rhs_lds(int ty, int lw, int nt) { return sizeof(double) * (size_t)std::max(X_NROWS * (ty + 2) * lw, nt); }
+
 
 // Number of z chunks over `tiles` workgroup tiles per plane range: at most
 // `want` (the launch's wavefront target), each at least `minpl` planes long.
@@ -1089,7 +1093,8 @@ static RhsShape rhs_shape(const ptc_ctx *c) {
   const int cols = kRhsSegThreads - 6, nseg = (c->nx + cols - 1) / cols;
   // 1.5 workgroups per CU with two-row segments and chunks of 16 planes
   const bool enough = 2LL * nseg * ((c->ny + 1) / 2) * std::max(1, c->nz / kRhsMinPlanes) >= 3LL * c->n_cu;
-  const bool whole = c->nx <= 128 || (c->nx > 2 * cols && c->nx <= 256) || (c->nx > 256 && c->nx <= 512 && !enough);
+  const bool whole = (c->nx <= 128 || (c->nx > 2 * cols && c->nx <= 256) || (c->nx > 256 && c->nx <= 512 && !enough)) &&
+                     rhs_lds(1, c->nx, 0) <= c->lds_limit;
   if (whole) {
     s.tx = (c->nx + 63) / 64 * 64;
     s.seg = 0;
@@ -1103,6 +1108,9 @@ static RhsShape rhs_shape(const ptc_ctx *c) {
   else ty = enough && sizeof(double) * c->n3 <= kRhsCachedField ? 2 : 4;
   if (c->rhs_rows_req) ty = c->rhs_rows_req;
   s.ty = std::max(1, std::min({ty, 512 / s.tx, c->ny}));
+  s.lw = s.seg ? s.tx : c->nx;
+  // (whole rows of 256 points take 74 KB for two, of 512 points 111 KB for one)
+  while (s.ty > 1 && rhs_lds(s.ty, s.lw, s.tx * s.ty) > c->lds_limit) --s.ty;
   s.run = c->rhs_run_req ? c->rhs_run_req : kRhsXcdRun;
   s.nseg = s.seg ? (c->nx + s.seg - 1) / s.seg : 1;
   s.nyb = (c->ny + s.ty - 1) / s.ty;
@@ -1119,6 +1127,10 @@ void rhs_shape_in_use(const ptc_ctx *c, int *seg_threads, int *rows, int *run, i
   *rows = s.ty;
   *run = s.run;
   *min_planes = s.minpl;
+}
+size_t rhs_lds_in_use(const ptc_ctx *c) {
+  const RhsShape s = rhs_shape(c);
+  return rhs_lds(s.ty, s.lw, s.tx * s.ty);
 }
 static dim3 rhs_rows_grid(const ptc_ctx *c, int *kc) {
   const RhsShape sh = rhs_shape(c);
@@ -1184,11 +1196,10 @@ int launch_rhs(ptc_ctx *c, const double *ux, const double *uy, const double *uz,
   const dim3 grid = rhs_rows_grid(c, &kc);
   const RhsShape sh = rhs_shape(c);
   const int nt = sh.tx * sh.ty;
-  const int lw = sh.seg ? sh.tx : c->nx;  // LDS row width
-  const size_t lds = sizeof(double) * (size_t)std::max(X_NROWS * (sh.ty + 2) * lw, nt);
+  const size_t lds = rhs_lds_in_use(c);
 #define PTC_ROWS(SCAL, MAXT, ONE)                                                                             \
   hipLaunchKernelGGL((k_rhs_rows<SCAL, MAXT, ONE>), grid, dim3(sh.tx, sh.ty), lds, c->stream, c->geo, cf, kc, ux, uy, \
-                     uz, sc, p, rhsx, rhsy, rhsz, rhsc, hx, hy, hz, hc, c->d_red, sh.seg, lw, sh.run)
+                     uz, sc, p, rhsx, rhsy, rhsz, rhsc, hx, hy, hz, hc, c->d_red, sh.seg, sh.lw, sh.run)
   if (sh.ty == 1) {
     if (cf.scalar) PTC_ROWS(true, 512, true);
     else PTC_ROWS(false, 512, true);

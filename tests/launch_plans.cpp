@@ -28,5 +28,23 @@ int main() {
       const bool ok = ptc::fft_x_shape(L, 65536, limit, &lines, &threads, &pad, &bytes);
       std::printf("x %d %zu %d %d %d %d %d %zu\n", h, limit, ok, L.threads, lines, threads, pad, bytes);
     }
+  // rhs: nx, ny, requested segment threads and rows, LDS limit, threads per row, rows, bytes
+  for (size_t limit : {size_t(65536), lds})
+    for (int nx = 8; nx <= 1100; nx += 2)
+      for (int ny : {4, 10, 96, 256})
+        for (int seg : {0, 64, 128, 256})
+          for (int rows : {0, 1, 2, 4, 8}) {
+            ptc_ctx c;
+            c.nx = nx;
+            c.ny = ny;
+            c.nz = 64;
+            c.n3 = (size_t)nx * (ny + 2) * c.nz;
+            c.lds_limit = limit;
+            c.rhs_seg_req = seg;
+            c.rhs_rows_req = rows;
+            int tx = 0, ty = 0, run = 0, minpl = 0;
+            ptc::rhs_shape_in_use(&c, &tx, &ty, &run, &minpl);
+            std::printf("rhs %d %d %d %d %zu %d %d %zu\n", nx, ny, seg, rows, limit, tx, ty, ptc::rhs_lds_in_use(&c));
+          }
   return 0;
 }

@@ -57,3 +57,14 @@ def test_run_time_x_lines_fit_the_lds_they_ask_for(plans):
             line = h + (h >> pad) + 1
             assert nbytes >= 16 * lines * line and nbytes >= 8 * threads, (h, nbytes)
     assert seen[65536] == seen[163840] and {3375, 3675, 4096} <= seen[65536]
+
+
+def test_rhs_rows_fit_the_lds(plans):
+    """The RHS kernel's rows (nine quantities, the workgroup's rows and two
+    ghost rows each) fit the device's LDS for every row length and request;
+    gfx950's limit takes no row away from a shape."""
+    for nx, ny, seg, rows, limit, tx, ty, nbytes in plans["rhs"]:
+        assert nbytes <= limit and 1 <= ty <= ny and tx * ty <= 512, (nx, ny, seg, rows, limit, nbytes)
+        assert nbytes >= 8 * 9 * (ty + 2) * min(nx, tx), (nx, ny, seg, rows, nbytes)
+        if limit == 163840 and rows:
+            assert ty == max(1, min(rows, 512 // tx, ny)), (nx, ny, seg, rows)
