@@ -787,8 +787,8 @@ static const TriShape kPoissonShapes[] = {{4, 64, 1024}, {8, 64, 1024}, {12, 64,
 // 512 threads for ny = 96, three workgroups per CU where 8-row chunks' 768 threads
 // leave a round of workgroups half empty (RK substep 128x96x128 144.8 -> 139.3 us,
 // 256x128x192 486 -> 472, 280x76x210 423 -> 413); above 192 rows chunks of 16
-// (64x256x64 114 -> 112).
-static const TriShape kCnShapes[] = {{12, 64, 1024}, {8, 64, 1024}, {4, 64, 1024}, {16, 32, 512}, {8, 32, 1024}};
+// (64x256x64 114 -> 112).  Every height up to 256 takes one of the four.
+static const TriShape kCnShapes[] = {{12, 64, 1024}, {8, 64, 1024}, {4, 64, 1024}, {16, 32, 512}};
 
 static int tri_choose(int ny, size_t lds_limit, int mm_req, int lpb_req, const TriShape *shapes, int nshapes,
                       int *P_out, int *mm_out, int *lpb_out) {
@@ -862,7 +862,7 @@ int tri_plan_cplx(int ny, size_t lds_limit, int cl, int mm_req, int *P_out, int 
 int tri_plan(int ny, size_t lds_limit, bool poisson, int mm_req, int lpb_req, int *P_out, int *mm_out,
              int *lpb_out) {
   return poisson ? tri_choose(ny, lds_limit, mm_req, lpb_req, kPoissonShapes, 8, P_out, mm_out, lpb_out)
-                 : tri_choose(ny, lds_limit, mm_req, lpb_req, kCnShapes, 5, P_out, mm_out, lpb_out);
+                 : tri_choose(ny, lds_limit, mm_req, lpb_req, kCnShapes, 4, P_out, mm_out, lpb_out);
 }
 
 int launch_tri_poisson(ptc_ctx *c, void *spec) {
@@ -1013,7 +1013,6 @@ static int launch_cn(ptc_ctx *c, const CnJobs &jobs, bool factor, bool solve, co
   PTC_CN(4, 64)
   PTC_CN(8, 64)
   PTC_CN(12, 64)
-  PTC_CN(8, 32)
   PTC_CN(16, 32)
 #undef PTC_CN
   set_error("bad tridiagonal launch shape");

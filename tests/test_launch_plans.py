@@ -43,6 +43,19 @@ def test_flow_rate_sum_exchanges_among_lanes_of_the_workgroup(plans):
     assert halves == 32  # ny 193-208 and 225-240
 
 
+def test_crank_nicolson_plan_of_every_height(plans):
+    """Every height up to 256 has a plan of one of the four compiled shapes, each
+    of which some height takes, within its launch bound and the factor table."""
+    cap = {(12, 64): 1024, (8, 64): 1024, (4, 64): 1024, (16, 32): 512}
+    assert {(p[2], p[3]) for p in plans["cn"]} == set(cap)
+    for ny, chunks, rows, lanes, _ in plans["cn"]:
+        assert chunks == -(-ny // rows) and chunks * lanes <= cap[rows, lanes], ny
+        assert chunks * rows <= 256 and 2 * chunks <= 64, ny
+    # the two sides of each change of shape
+    by_ny = {p[0]: (p[2], p[3], p[1]) for p in plans["cn"]}
+    assert by_ny[192] == (12, 64, 16) and by_ny[193] == (16, 32, 13) and by_ny[256] == (16, 32, 16)
+
+
 def test_run_time_x_lines_fit_the_lds_they_ask_for(plans):
     """Every line up to 4096 values has a launch on gfx950, and no accepted
     launch asks for more LDS than the limit or than its kernels' last slot
