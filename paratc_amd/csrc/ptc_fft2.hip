@@ -315,11 +315,12 @@ constexpr int f2_x_min_waves() {
 // The residual-forming form holds twenty more loads per point pair: held to
 // those bounds it spills 96-188 bytes per lane, so it takes the registers it
 // needs (three waves per SIMD at most).
-// The divergence by columns of 512- and 1024-point rows is held to 128 VGPRs (it
-// takes 130 left alone).
+// The divergence by columns takes 130 VGPRs at 512-point rows and 117 at 1024 and
+// is left alone: held to 128 the former spilled 7 and was slower (a step of
+// 512x128x256 3736 us against 3721, 512x96x128 1429 against 1415).
 template <int N, int SRC>
 constexpr int f2_xfwd_min_waves() {
-  return SRC >= 2 ? ((N == 2304 || N == 4608) ? 3 : 1) : (SRC == 1 && N >= 256 && N <= 512 ? 4 : f2_x_min_waves<N>());
+  return SRC >= 2 ? ((N == 2304 || N == 4608) ? 3 : 1) : f2_x_min_waves<N>();
 }
 // Planes a thread takes at a time where the divergence is formed by columns
 // (1: pair by pair), and the lines of a workgroup then, whole groups of them.
