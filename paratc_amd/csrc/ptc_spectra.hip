@@ -36,7 +36,13 @@ namespace ptc {
 
 namespace {
 
-constexpr int kSpecThreads = 320;  // largest partial-sum workgroup: 257 kx (nx = 512) fit one per thread
+// Largest partial-sum workgroup.  With 320 threads the 2^k + 1 kx of a power of two
+// fit fewer kx per thread (257 one, 513 two), but two loads per thread in flight
+// serve better than one: a sample (us, 256 / 320 threads) of 512x128x256 599 / 650,
+// 512x96x192 384 / 409, 540x96x128 312 / 331, 600x64x128 251-256 / 259, 1024x128x192
+// 858 / 868; the other way 512x32x64 136 / 130, 1024x64x128 343 / 334; 250 to 400 and
+// 768 to 2048 points otherwise within 1 %, 384 and 512 threads as 320.
+constexpr int kSpecThreads = 256;
 constexpr size_t kSpecStage = size_t(2) << 20;  // bytes of a pinned half
 constexpr int kSpecRows = 16;      // kz rows per partial-sum workgroup
 
