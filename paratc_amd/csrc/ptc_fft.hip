@@ -17,16 +17,19 @@
 // radix plan at run time.  Every stage of a line has one butterfly per thread:
 // its R inputs are loaded, transformed by a DFT whose radix is a compile-time
 // constant (a switch on the plan's radix, uniform over the launch) and stored,
-// all in registers, so no private memory is touched; the first stage reads HBM
+// in registers (two forms of workgroups of up to 1024 threads, held to 128
+// VGPRs, spill: radix 15, 24-25 of them, for lines of 3375 and 3675 values only,
+// and the x pass that forms the source in lines of more than 256 threads, 160:
+// see poisson_div_fusable); the first stage reads HBM
 // and the last one writes it, LDS carries the exchanges between them.  A line
 // takes G = n / (smallest radix) threads; radices of 2 to 10 with as few and
 // as even factors as the length allows (fft_make_len) keep the threads busy in
 // every stage: 150 = 6 * 5 * 5, 180 = 6 * 6 * 5, 90 = 10 * 9.  The division
-// by the span of a stage is a multiplication with a 32-bit reciprocal.  Bound by
-// memory: at 360 x 90 x 150 (78 MB moved per pass) the four passes take about
-// 12 us each, 6 TB/s out of the last-level cache, where kernels that staged
-// several run-time butterflies per thread in private memory took 51-55 us
-// (solve 214 -> 74 us).
+// by the span of a stage is a multiplication with a 32-bit reciprocal.  At
+// 360 x 90 x 150 (80 MB moved per pass, all of it in the last-level cache, whence a
+// copy of that size moves 6.8 TB/s) the four passes take 23-25 us each, 3.3 TB/s,
+// at three to four waves per SIMD, where kernels that staged several run-time
+// butterflies per thread in private memory took 52-55 us (solve 221 -> 102 us).
 #include <cmath>
 #include <cstring>
 

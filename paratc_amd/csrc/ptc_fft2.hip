@@ -336,7 +336,7 @@ constexpr int f2_div_lines() {
 }
 // Lines of one plane column in the column form of the residual (kXResCol), or
 // 0 where the length has none: a workgroup's lines in groups of K consecutive
-// planes of one row, N * lines a multiple of K * 256.
+// planes of one row, N * lines a multiple of K times the threads (f2_xbase).
 template <int N>
 constexpr int f2_res_lines() {
   constexpr int L = f2_threads<N>() <= f2_xbase<N>() ? f2_xbase<N>() / f2_threads<N>() : 1;
@@ -366,7 +366,7 @@ constexpr int f2_res_lines() {
 constexpr int kXPlain = 0, kXDiv = 1, kXRes = 2, kXResCol = 3;
 
 // The residual of a workgroup's lines q0 .. q0+L-1 into their LDS rows (the
-// column form).  Each thread takes the columns threadIdx.x + 256 c: pair m of
+// column form).  Each thread takes the columns threadIdx.x + f2_xbase c: pair m of
 // the K planes of one group of lines.  All the planes of its columns are in
 // flight at once, then the rows above and below and f, one column after the
 // other; edge rows load their own row for the missing one (the Neumann

@@ -302,7 +302,14 @@ int poisson_solve(ptc_ctx *c, const double *src, double *dst, bool ghosts) {
 bool poisson_div_fusable(ptc_ctx *c) {
   if (poisson_build_plan(c) != PTC_OK) return false;
   const PoissonPlan &P = c->pp;
-  // (a run-time length plan with a radix above 10 has no registers left for it)
+  // A run-time length plan with a radix above 10 has no such form: its plain one
+  // spills already.  Lines of more than 256 threads (nx = 1372, most above 2048) have
+  // it though it spills at its 128 VGPRs (180 B a lane): a step is
+  // within 3 % of k_prsrc and the plain pass either way (us, in the pass /
+  // separate: 1372x96x96 3705 / 3607, 2304x64x96 3742 / 3646, 3072x96x128 9383 /
+  // 9373, 4096x64x64 3983 / 4066, 4096x96x128 11480 / 11830, 6000x64x64 6382 /
+  // 6316, 8192x48x64 5997 / 6157), and in workgroups of 512 threads at 168
+  // VGPRs, without spills, took 3811, 3899, 9497 and 4049 at the first four.
   return P.slab == 0 && P.prec == PTC_PREC_FP64 && (P.x_fast || P.fx.radix[0] <= 10);
 }
 

@@ -1043,13 +1043,14 @@ static int pt_nblocks(const ptc_ctx *c) {
 //   <= 128: whole rows, two (128x96x128: 42 / 55 against 47 / 63 with four);
 //   <= 244: two segments of 128 threads, two rows: four wavefronts, so two
 //     workgroups share a CU (240x64x96: 42 / 56 against 47 / 65 for whole rows;
-//     192x96x128: 66 / 85 against 63 / 100);
+//     192x96x128: 66 / 85 against 63 / 100: of the rows measured the one where
+//     whole rows win, by 5 % and without the scalar only, so one rule serves both);
 //   <= 256: whole rows, two (256x128x192: 158 / 215 against 200 / 264, three
 //     segments would idle a third of the lanes);
 //   <= 512: segments of 128 threads, two rows (280x76x210: 137 / 187 against 197
 //     / 304 for whole rows, 512x128x256: 458 / 618 against 464 / 908), or whole
 //     rows, one per workgroup, where the grid is too small for 1.5 such
-//     workgroups per CU;
+//     workgroups per CU (with the scalar that form spills 9 of 256 VGPRs);
 //   longer: segments of 128 threads; two rows while a field fits the last-level
 //     cache (1024x128x160: 533 / 731 against 587 / 778 with four; 768x128x192:
 //     497 / 674 against 545 / 711), four beyond it, where the re-read edge rows
@@ -1525,8 +1526,9 @@ namespace ptc {
 // ahead, and the x neighbours (the z difference of uy that dvdzC interpolates
 // included) go through LDS rows, double-buffered so that a plane takes one
 // barrier.  Twelve loads per point instead of about ninety: bound by the loads'
-// latency at the two wavefronts per SIMD that the 40 running sums leave
-// (256x128x192 with a scalar: 563 us a sample before, about 115 now).  part[(j-1) nparts + part][NS]
+// latency at the two wavefronts per SIMD that the running sums leave (248
+// VGPRs; 256 and 4 spilled with the scalar's 40 sums; 256x128x192 with a scalar:
+// 563 us a sample before, 113 now, 99 without).  part[(j-1) nparts + part][NS]
 // with part = segment * nch + chunk.  The last row group of the grid is the top
 // wall face j = ny+1, which has only the terms 27, 33 and 35 (1-based).
 enum { T_U = 0, T_V, T_VP, T_W, T_P, T_PM, T_C4, T_NROWS };

@@ -153,8 +153,10 @@ __device__ __forceinline__ void chunk_backsub(V (&f)[MM], const double (&A)[MM],
 // neighbours p-d and p+d, so after ceil(log2 P) steps each row stands alone;
 // the first value then follows from its row.  (All 2P rows through the
 // reduction took one more step and twice the rows a step: the y pass of
-// 1024x256x512 with FP32 spectra 343 us, now 253; a solve of 128x96x128 51.8,
-// now 49.8; errors against the oracle as before or smaller.)  Rows outside the
+// 1024x256x512 with FP32 spectra 328 us, now 247; a solve of 128x96x128 51.8,
+// now 49.8.  FP64 solution errors against 64 bits at equal chunk length, 48 to 256
+// rows: at most 3 % larger, up to 7 % smaller, most within 1 %; the chunk length
+// moves them by up to a factor of five.)  Rows outside the
 // system act as decoupled identity rows.  They live in LDS, double-buffered ([2][P][LPB]
 // for each of a, c, f): a step reads one buffer and writes the other, so it
 // needs one barrier and holds nothing in registers across steps.  The reference
