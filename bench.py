@@ -247,11 +247,11 @@ def bench_spectra(r, ev, samples=5):
     ms = ev.elapsed_ms(e0, e1) / samples
     _, _, _, n = s.get_spectra(reset=True)
     assert n == samples + 1
-    # per point: the cell-centre uy (8 B read + 8 B write), five FP64 forward
-    # transforms (ux, uy, uz, p, cell-centre uy; x and z pass, 8 B read + 8 B
-    # write each; the cell-centre ux spectrum is formed from the ux one), and
-    # the partial sums reading nine spectra (8 B per point each)
-    alg = 16 + 5 * 32 + 9 * 8
+    # per point: four FP64 forward transforms (ux, uy, uz, p; x and z pass, 8 B
+    # read + 8 B write each; the cell-centre ux and uy spectra are formed from
+    # theirs), and the partial sums reading each spectrum once (8 B per point),
+    # uy's twice (its energy, and with ux's products)
+    alg = 4 * 32 + 5 * 8
     progress(f"spectra 1024x256x512: {ms:.3f} ms per sample")
     return {"workload": "clcStat energy spectra, 1-D (8 quantities) + 2-D (5 quantities, 4 rows), "
                         "1024x256x512 FP64", "ms_per_sample": round(ms, 3),
